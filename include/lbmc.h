@@ -132,7 +132,11 @@ lbmc_status lbmc_init_equilibrium(lbmc_ctx *ctx, const double *rho, const double
 lbmc_status lbmc_step(lbmc_ctx *ctx, long long t, int store_macros);
 
 /* nsteps calls with t = t0 .. t0+nsteps-1; macros are stored on the calls
- * where (t+1) % store_every == 0 (store_every <= 0: never). */
+ * where (t+1) % store_every == 0 (store_every <= 0: never).  Lattices whose
+ * calls the library runs several at a time (D2Q9 without sf boundaries) hold
+ * a second population array from lbmc_set_fields on, taken only while half
+ * of the device's memory stays free and given back when a later allocation
+ * of the library does not fit; the results do not depend on it. */
 lbmc_status lbmc_run(lbmc_ctx *ctx, long long t0, int nsteps, int store_every);
 
 /* As lbmc_run, timed with HIP events on the context's stream; *ms is the

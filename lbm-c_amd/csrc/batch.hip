@@ -277,10 +277,10 @@ lbmc_status build_chunks(lbmc_batch *b, int sub)
     if (b->cchunks) B_HIP(b, hipFree(b->cchunks));
     b->chunks = nullptr;
     b->cchunks = nullptr;
-    B_HIP(b, hipMalloc((void **)&b->chunks, sizeof(int2) * ch.size()));
+    B_HIP(b, dev_malloc((void **)&b->chunks, sizeof(int2) * ch.size()));
     B_HIP(b, hipMemcpy(b->chunks, ch.data(), sizeof(int2) * ch.size(), hipMemcpyHostToDevice));
     if (!cc.empty()) {
-        B_HIP(b, hipMalloc((void **)&b->cchunks, sizeof(int2) * cc.size()));
+        B_HIP(b, dev_malloc((void **)&b->cchunks, sizeof(int2) * cc.size()));
         B_HIP(b, hipMemcpy(b->cchunks, cc.data(), sizeof(int2) * cc.size(), hipMemcpyHostToDevice));
     }
     b->nchunks = (int)ch.size();
@@ -374,9 +374,9 @@ lbmc_status lbmc_batch_create(lbmc_ctx *const *members, int count, lbmc_batch **
     if (e == hipSuccess) e = hipEventCreate(&b->ev0);
     if (e == hipSuccess) e = hipEventCreate(&b->ev1);
     const size_t msz = b->cdouble ? sizeof(BatchMember<double>) : sizeof(BatchMember<float>);
-    if (e == hipSuccess) e = hipMalloc(&b->dmembers, msz * (size_t)count);
-    if (e == hipSuccess) e = hipMalloc(&b->dwindow, msz * (size_t)count * kBatchWindow);
-    if (e == hipSuccess) e = hipMalloc((void **)&b->any_eval, sizeof(int) * kBatchWindow);
+    if (e == hipSuccess) e = dev_malloc(&b->dmembers, msz * (size_t)count);
+    if (e == hipSuccess) e = dev_malloc(&b->dwindow, msz * (size_t)count * kBatchWindow);
+    if (e == hipSuccess) e = dev_malloc((void **)&b->any_eval, sizeof(int) * kBatchWindow);
     if (e != hipSuccess) return bail(bfail(b, LBMC_ERR_DEVICE, "lbmc_batch_create: %s", hipGetErrorString(e)));
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, b->device) == hipSuccess && prop.multiProcessorCount > 0)

@@ -5,10 +5,12 @@
 #include <hip/hip_runtime.h>
 
 #include <cstring>
+#include <mutex>
 #include <string>
 
 #include "../../include/lbmc.h"
 #include "step_args.hpp"
+#include "tile_pass.hpp"
 
 struct lbmc_ctx {
     lbmc_desc desc{};
@@ -59,6 +61,15 @@ struct lbmc_ctx {
     double closure_shift = 0;  // added to the network's tau' on this lattice
     float *tcache = nullptr;
     bool tcache_valid = false;
+
+    // passes of several calls (tile_kernel.hpp): tile shape, and the second
+    // population buffer that they write to (null: one call per launch).
+    // pass_mu: held while launches that use f2 are issued, and by another
+    // thread that takes f2 back when device memory runs out (dev_malloc)
+    lbmc::TilePlan tile{};
+    void *f2 = nullptr;
+    std::mutex pass_mu;
+    bool has_macro = false;  // some node prescribes rho or u from the macro arrays
 
     // launch shape
     int grid = 1;

@@ -9,14 +9,29 @@
 
 #include "../../include/lbmc.h"
 #include "step_args.hpp"
+#include "tile_pass.hpp"
 
 namespace lbmc {
+
+// hipMalloc on the current device; when memory runs out, the second
+// population buffers of its lattices are given back and it is tried again
+hipError_t dev_malloc(void **p, size_t bytes);
 
 // fused step, step_<storage>.hip
 hipError_t launch_step_fp64(const KernelKey &k, const StepArgs<double> &a, int grid, hipStream_t s);
 hipError_t launch_step_fp32(const KernelKey &k, const StepArgs<float> &a, int grid, hipStream_t s);
 hipError_t launch_step_fp16s(const KernelKey &k, const StepArgs<float> &a, int grid, hipStream_t s);
 hipError_t launch_step_bf16s(const KernelKey &k, const StepArgs<float> &a, int grid, hipStream_t s);
+
+// several calls of a D2Q9 lattice in one pass, tile_<storage>.hip
+hipError_t launch_tile_fp64(const KernelKey &k, int size, const StepArgs<double> &a, const TilePass &p, int tiles,
+                            hipStream_t s);
+hipError_t launch_tile_fp32(const KernelKey &k, int size, const StepArgs<float> &a, const TilePass &p, int tiles,
+                            hipStream_t s);
+hipError_t launch_tile_fp16s(const KernelKey &k, int size, const StepArgs<float> &a, const TilePass &p, int tiles,
+                             hipStream_t s);
+hipError_t launch_tile_bf16s(const KernelKey &k, int size, const StepArgs<float> &a, const TilePass &p, int tiles,
+                             hipStream_t s);
 
 // sf neighbour gather, step_<storage>.hip
 hipError_t launch_sf_gather_fp64(int lattice, const StepArgs<double> &a, const int *sfnb, int nsf,

@@ -180,6 +180,66 @@ void choose_shape(lbmc_ctx *c)
     c->reuse_grid = (int)row_grid((unsigned)chunks, c->rlog);
 }
 
+// Lattices that hold a second population buffer
+std::mutex g_pass_mu;
+std::vector<lbmc_ctx *> g_pass_ctx;
+
+// Back to one call per launch (pass_mu held, or no other user)
+void drop_passes(lbmc_ctx *c)
+{
+    {
+        std::lock_guard<std::mutex> lock(g_pass_mu);
+        g_pass_ctx.erase(std::remove(g_pass_ctx.begin(), g_pass_ctx.end(), c), g_pass_ctx.end());
+    }
+    c->tile = TilePlan{};
+    free_dev(c->f2);
+}
+
+// Tiles of the passes over a lattice and their second population buffer:
+// D2Q9 lattices without sf nodes whose direction arrays 32-bit offsets
+// reach.  The buffer is taken only while half of the device's memory stays
+// free, and given back when an allocation fails (dev_malloc), so that a
+// program's lattices fit as they would without it.
+void plan_passes(lbmc_ctx *c)
+{
+    std::lock_guard<std::mutex> lock(c->pass_mu);
+    TilePlan q;
+    if (c->D == 2 && !c->nsf && !c->offsets64) {
+        int ncu = 256;
+        (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->desc.device);
+        q = plan_tiles(c->L[0], c->L[1], (int)c->sbytes, std::max(1, ncu));
+        // test hook: LBMC_PASS=0 one call per launch, or "size,W,H,M" a tile shape
+        if (const char *env = getenv("LBMC_PASS")) {
+            int v[4] = {0, 0, 0, 0};
+            q = TilePlan{};
+            if (sscanf(env, "%d,%d,%d,%d", &v[0], &v[1], &v[2], &v[3]) == 4 && v[0] >= 0 && v[0] <= 2 && v[3] >= 0 &&
+                v[3] < 32) {
+                const TileCapacity cap = tile_capacity(v[0], (int)c->sbytes);
+                q.on = (long long)v[1] * v[2] <= cap.threads * cap.per_thread &&
+                       tile_shape(c->L[0], c->L[1], v[0], v[1], v[2], v[3], q);
+            }
+        }
+    }
+    if (!q.on) {
+        drop_passes(c);
+        return;
+    }
+    if (!c->f2) {
+        const size_t bytes = c->sbytes * (size_t)c->Q * (size_t)c->npad;
+        size_t avail = 0, total = 0;
+        if (hipMemGetInfo(&avail, &total) != hipSuccess || avail < bytes + total / 2 ||
+            hipMalloc(&c->f2, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            c->f2 = nullptr;
+            drop_passes(c);
+            return;
+        }
+        std::lock_guard<std::mutex> g(g_pass_mu);
+        g_pass_ctx.push_back(c);
+    }
+    c->tile = q;
+}
+
 void drop_graph(lbmc_ctx *c)
 {
     if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
@@ -209,6 +269,81 @@ long long lcm_ll(long long a, long long b)
     return a / x * b;
 }
 
+// One pass of `calls` calls from t: src -> dst.  A pass that starts or ends a
+// run reads or leaves the stored layout (slots shifted by the call); between
+// passes the buffers hold every node's post-collision values at the node
+// itself.
+template <class C>
+hipError_t launch_pass(lbmc_ctx *c, long long t, int calls, unsigned store, bool first, bool last, const void *src,
+                       void *dst)
+{
+    StepArgs<C> a;
+    fill_args(c, a, t, 0);
+    TilePass p;
+    memset(&p, 0, sizeof(p));
+    tile_geometry(c->tile, c->L, p);
+    p.src = src;
+    p.dst = dst;
+    p.calls = calls;
+    p.store = store;
+    for (int d = 0; d < 2; d++) {
+        p.s0[d] = a.s[d];
+        p.rs[d] = first ? a.s[d] : 1 % c->L[d];
+        p.ws[d] = last ? (int)((t + calls - 1) % c->L[d]) : 0;
+    }
+    const int tiles = c->tile.ntx * c->tile.nty;
+    if constexpr (sizeof(C) == 8) {
+        return launch_tile_fp64(c->key, c->tile.size, a, p, tiles, c->stream);
+    } else {
+        switch (c->storage) {
+        case LBMC_FP32: return launch_tile_fp32(c->key, c->tile.size, a, p, tiles, c->stream);
+        case LBMC_FP16S: return launch_tile_fp16s(c->key, c->tile.size, a, p, tiles, c->stream);
+        default: return launch_tile_bf16s(c->key, c->tile.size, a, p, tiles, c->stream);
+        }
+    }
+}
+
+// len >= 2 calls from t: an even number of passes, so that the state ends in
+// the buffer it started in
+lbmc_status run_passes(lbmc_ctx *c, long long t, long long len, int store_every)
+{
+    const int K = c->tile.M + 1;
+    const long long np = 2 * ((len + 2 * K - 1) / (2 * K));
+    for (long long k = 0; k < np; k++) {
+        const long long k0 = len * k / np, k1 = len * (k + 1) / np;
+        unsigned store = 0;
+        for (long long j = k0; j < k1; j++)
+            if (store_every > 0 && (t + j + 1) % store_every == 0) store |= 1u << (j - k0);
+        const void *src = k & 1 ? c->f2 : c->f;
+        void *dst = k & 1 ? c->f : c->f2;
+        const hipError_t e =
+            c->cbytes == 8 ? launch_pass<double>(c, t + k0, (int)(k1 - k0), store, k == 0, k + 1 == np, src, dst)
+                           : launch_pass<float>(c, t + k0, (int)(k1 - k0), store, k == 0, k + 1 == np, src, dst);
+        if (e != hipSuccess) return hip_fail(c, e, "pass launch");
+    }
+    return LBMC_OK;
+}
+
+// Calls t .. t + nsteps - 1 in passes.  Calls that store the macros of a
+// lattice with prescribed values run alone: the stored arrays are also what
+// the next call prescribes, and a pass's tiles read them at different times.
+lbmc_status run_in_passes(lbmc_ctx *c, long long t, int nsteps, int store_every)
+{
+    const long long end = t + nsteps;
+    while (t < end) {
+        long long e = end;
+        if (c->has_macro && store_every > 0) e = std::min(end, (t + store_every) / store_every * store_every - 1);
+        if (e - t >= 2) {
+            if (lbmc_status st = run_passes(c, t, e - t, store_every)) return st;
+            t = e;
+        } else {
+            if (lbmc_status st = launch_step(c, t, store_every > 0 && (t + 1) % store_every == 0)) return st;
+            t++;
+        }
+    }
+    return LBMC_OK;
+}
+
 // The kernel arguments of call t depend on t only through t mod L_d and,
 // for the macro store, (t + 1) mod store_every.  A run of P = lcm of those
 // calls therefore repeats exactly: capture it once into a graph and replay.
@@ -220,6 +355,10 @@ lbmc_status run_steps(lbmc_ctx *c, long long t0, int nsteps, int store_every)
         if (lbmc_status st = launch_step(c, t0, store_every > 0 && ((t0 + 1) % store_every) == 0)) return st;
         t0++;
         nsteps--;
+    }
+    {
+        std::lock_guard<std::mutex> lock(c->pass_mu);
+        if (c->tile.on && !c->key.closure) return run_in_passes(c, t0, nsteps, store_every);
     }
     auto stores = [&](long long tt) { return store_every > 0 && ((tt + 1) % store_every) == 0; };
     long long period = lcm_ll(lcm_ll(c->L[0], c->L[1]), c->L[2]);
@@ -264,6 +403,38 @@ lbmc_status run_steps(lbmc_ctx *c, long long t0, int nsteps, int store_every)
 }
 
 }  // namespace
+
+namespace lbmc {
+
+hipError_t dev_malloc(void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return e;
+    bool freed = false;
+    {
+        std::lock_guard<std::mutex> lock(g_pass_mu);
+        for (size_t k = 0; k < g_pass_ctx.size();) {
+            lbmc_ctx *c = g_pass_ctx[k];
+            // a lattice whose launches are being issued keeps its buffer
+            if (c->desc.device != dev || !c->pass_mu.try_lock()) {
+                k++;
+                continue;
+            }
+            (void)hipStreamSynchronize(c->stream);
+            c->tile = TilePlan{};
+            free_dev(c->f2);
+            g_pass_ctx.erase(g_pass_ctx.begin() + (long)k);
+            c->pass_mu.unlock();
+            freed = true;
+        }
+    }
+    (void)hipGetLastError();
+    return freed ? hipMalloc(p, bytes) : e;
+}
+
+}  // namespace lbmc
 
 extern "C" {
 
@@ -371,20 +542,20 @@ lbmc_status lbmc_create(const lbmc_desc *desc, lbmc_ctx **out)
     }
     if ((e = hipEventCreate(&c->ev0)) != hipSuccess || (e = hipEventCreate(&c->ev1)) != hipSuccess)
         return bail(hip_fail(c, e, "hipEventCreate"));
-    if ((e = hipMalloc(&c->f, c->sbytes * (size_t)c->Q * (size_t)c->npad)) != hipSuccess)
+    if ((e = dev_malloc(&c->f, c->sbytes * (size_t)c->Q * (size_t)c->npad)) != hipSuccess)
         return bail(hip_fail(c, e, "populations"));
-    if ((e = hipMalloc((void **)&c->mask, (size_t)c->npad)) != hipSuccess)
+    if ((e = dev_malloc((void **)&c->mask, (size_t)c->npad)) != hipSuccess)
         return bail(hip_fail(c, e, "node mask"));
-    if ((e = hipMalloc((void **)&c->cls, 256 * sizeof(uint16_t))) != hipSuccess)
+    if ((e = dev_malloc((void **)&c->cls, 256 * sizeof(uint16_t))) != hipSuccess)
         return bail(hip_fail(c, e, "class table"));
-    if ((e = hipMalloc(&c->rho, c->cbytes * (size_t)c->npad)) != hipSuccess)
+    if ((e = dev_malloc(&c->rho, c->cbytes * (size_t)c->npad)) != hipSuccess)
         return bail(hip_fail(c, e, "rho"));
     for (int d = 0; d < 3; d++)
-        if ((e = hipMalloc(&c->u[d], c->cbytes * (size_t)c->npad)) != hipSuccess)
+        if ((e = dev_malloc(&c->u[d], c->cbytes * (size_t)c->npad)) != hipSuccess)
             return bail(hip_fail(c, e, "u"));
     c->npartials = 1024;
-    if ((e = hipMalloc((void **)&c->partials, sizeof(double) * c->npartials)) != hipSuccess ||
-        (e = hipMalloc((void **)&c->scalar, sizeof(double))) != hipSuccess)
+    if ((e = dev_malloc((void **)&c->partials, sizeof(double) * c->npartials)) != hipSuccess ||
+        (e = dev_malloc((void **)&c->scalar, sizeof(double))) != hipSuccess)
         return bail(hip_fail(c, e, "reduction scratch"));
     // zero state: plain fluid everywhere, zero macros, zero populations
     if ((e = hipMemset(c->mask, 0, (size_t)c->npad)) != hipSuccess ||
@@ -405,6 +576,10 @@ lbmc_status lbmc_destroy(lbmc_ctx *c)
     if (!c) return LBMC_OK;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     drop_graph(c);
+    {
+        std::lock_guard<std::mutex> lock(c->pass_mu);
+        drop_passes(c);
+    }
     free_dev(c->f);
     void *p;
     p = c->mask; free_dev(p); c->mask = nullptr;
@@ -486,6 +661,10 @@ lbmc_status lbmc_set_fields(lbmc_ctx *c, const double *geometry, const int *macr
         all_fluid = all_fluid && maskv[(size_t)n] == 0;
     }
     c->all_fluid = all_fluid;
+    {
+        std::lock_guard<std::mutex> lock(c->pass_mu);
+        c->tile = TilePlan{};  // planned again for the new fields below
+    }
     HIP_TRY(c, hipMemcpy(c->mask, maskv.data(), (size_t)N, hipMemcpyHostToDevice), "mask upload");
     HIP_TRY(c, hipMemcpy(c->cls, table, sizeof(table), hipMemcpyHostToDevice), "class upload");
     memcpy(c->cls_host, table, sizeof(table));
@@ -495,7 +674,7 @@ lbmc_status lbmc_set_fields(lbmc_ctx *c, const double *geometry, const int *macr
     free_dev(c->porosity);
     c->porous = any_porous;
     if (any_porous) {
-        HIP_TRY(c, hipMalloc(&c->porosity, c->cbytes * (size_t)c->npad), "porosity");
+        HIP_TRY(c, dev_malloc(&c->porosity, c->cbytes * (size_t)c->npad), "porosity");
         std::vector<double> b(geometry, geometry + N);
         if (lbmc_status st = upload_c(c, c->porosity, b)) return st;
     }
@@ -523,7 +702,7 @@ lbmc_status lbmc_set_fields(lbmc_ctx *c, const double *geometry, const int *macr
             for (int d = 0; d < 3; d++) c->F[d] = F0[d];
         } else {
             for (int d = 0; d < c->D; d++) {
-                HIP_TRY(c, hipMalloc(&c->force[d], c->cbytes * (size_t)c->npad), "force");
+                HIP_TRY(c, dev_malloc(&c->force[d], c->cbytes * (size_t)c->npad), "force");
                 std::vector<double> v((size_t)N, 0.0);
                 if (force[d]) v.assign(force[d], force[d] + N);
                 if (lbmc_status st = upload_c(c, c->force[d], v)) return st;
@@ -562,12 +741,15 @@ lbmc_status lbmc_set_fields(lbmc_ctx *c, const double *geometry, const int *macr
             nb[s] = (int)(xyz[0] + (long long)xyz[1] * c->L[0] + (long long)xyz[2] * c->L[0] * c->L[1]);
             idx[(size_t)n] = s;
         }
-        HIP_TRY(c, hipMalloc((void **)&c->sfnb, sizeof(int) * c->nsf), "sf list");
-        HIP_TRY(c, hipMalloc((void **)&c->sfidx, sizeof(int) * (size_t)c->npad), "sf index");
-        HIP_TRY(c, hipMalloc(&c->sfbuf, c->cbytes * (size_t)c->Q * c->nsf), "sf buffer");
+        HIP_TRY(c, dev_malloc((void **)&c->sfnb, sizeof(int) * c->nsf), "sf list");
+        HIP_TRY(c, dev_malloc((void **)&c->sfidx, sizeof(int) * (size_t)c->npad), "sf index");
+        HIP_TRY(c, dev_malloc(&c->sfbuf, c->cbytes * (size_t)c->Q * c->nsf), "sf buffer");
         HIP_TRY(c, hipMemcpy(c->sfnb, nb.data(), sizeof(int) * c->nsf, hipMemcpyHostToDevice), "sf upload");
         HIP_TRY(c, hipMemcpy(c->sfidx, idx.data(), sizeof(int) * (size_t)N, hipMemcpyHostToDevice), "sf upload");
     }
+    c->has_macro = false;
+    for (int j = 1; j < k; j++) c->has_macro = c->has_macro || cls_macro(table[j]) != 0;
+    plan_passes(c);
     HIP_TRY(c, hipDeviceSynchronize(), "set_fields sync");
     c->tcache_valid = false;
     drop_graph(c);
@@ -591,7 +773,7 @@ lbmc_status lbmc_get_links(lbmc_ctx *c, uint16_t *links)
     if (!c || !links) return fail(c, LBMC_ERR_INVALID, "null argument");
     HIP_TRY(c, hipSetDevice(c->desc.device), "hipSetDevice");
     uint16_t *dl = nullptr;
-    HIP_TRY(c, hipMalloc((void **)&dl, sizeof(uint16_t) * (size_t)c->npad), "links");
+    HIP_TRY(c, dev_malloc((void **)&dl, sizeof(uint16_t) * (size_t)c->npad), "links");
     hipError_t e = launch_links(c->desc.lattice, c->mask, c->cls, c->L[0], c->L[1], c->L[2], dl, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e == hipSuccess) e = hipMemcpy(links, dl, sizeof(uint16_t) * (size_t)c->N, hipMemcpyDeviceToHost);
@@ -619,8 +801,8 @@ lbmc_status lbmc_init_equilibrium(lbmc_ctx *c, const double *rho, const double *
     HIP_TRY(c, hipSetDevice(c->desc.device), "hipSetDevice");
     const size_t nb = sizeof(double) * (size_t)c->N;
     double *dr = nullptr, *du[3] = {nullptr, nullptr, nullptr};
-    hipError_t e = hipMalloc((void **)&dr, nb);
-    for (int d = 0; d < c->D && e == hipSuccess; d++) e = hipMalloc((void **)&du[d], nb);
+    hipError_t e = dev_malloc((void **)&dr, nb);
+    for (int d = 0; d < c->D && e == hipSuccess; d++) e = dev_malloc((void **)&du[d], nb);
     if (e == hipSuccess) e = hipMemcpy(dr, rho, nb, hipMemcpyHostToDevice);
     for (int d = 0; d < c->D && e == hipSuccess; d++) e = hipMemcpy(du[d], u[d], nb, hipMemcpyHostToDevice);
     if (e == hipSuccess)
@@ -717,7 +899,7 @@ lbmc_status lbmc_get_f(lbmc_ctx *c, double *const *f)
     if (!c || !f) return fail(c, LBMC_ERR_INVALID, "null argument");
     HIP_TRY(c, hipSetDevice(c->desc.device), "hipSetDevice");
     double *tmp = nullptr;
-    HIP_TRY(c, hipMalloc((void **)&tmp, sizeof(double) * (size_t)c->N), "f read buffer");
+    HIP_TRY(c, dev_malloc((void **)&tmp, sizeof(double) * (size_t)c->N), "f read buffer");
     hipError_t e = hipSuccess;
     for (int i = 0; i < c->Q && e == hipSuccess; i++) {
         if (!f[i]) continue;
@@ -792,7 +974,7 @@ lbmc_status lbmc_set_f(lbmc_ctx *c, const double *const *f)
     invalidate_tau_record(c);
     HIP_TRY(c, hipSetDevice(c->desc.device), "hipSetDevice");
     double *tmp = nullptr;
-    HIP_TRY(c, hipMalloc((void **)&tmp, sizeof(double) * (size_t)c->N), "f write buffer");
+    HIP_TRY(c, dev_malloc((void **)&tmp, sizeof(double) * (size_t)c->N), "f write buffer");
     hipError_t e = hipStreamSynchronize(c->stream);
     for (int i = 0; i < c->Q && e == hipSuccess; i++) {
         if (!f[i]) continue;
@@ -836,7 +1018,7 @@ lbmc_status lbmc_set_closure(lbmc_ctx *c, const lbmc_mlp *model, double tau_lo, 
     if (!(tau_lo > 0.5) || !(tau_hi >= tau_lo) || !std::isfinite(tau_hi))
         return fail(c, LBMC_ERR_INVALID, "lbmc_set_closure: band [%g, %g] must satisfy 0.5 < lo <= hi", tau_lo, tau_hi);
     HIP_TRY(c, hipSetDevice(c->desc.device), "hipSetDevice");
-    if (!c->mlp_img) HIP_TRY(c, hipMalloc(&c->mlp_img, mlp_image_bytes()), "closure image allocation");
+    if (!c->mlp_img) HIP_TRY(c, dev_malloc(&c->mlp_img, mlp_image_bytes()), "closure image allocation");
     HIP_TRY(c, hipStreamSynchronize(c->stream), "closure sync");
     const lbmc_status st = mlp_build_image(model, c->mlp_img, c->desc.device, tau_lo, tau_hi, c->stream);
     if (st != LBMC_OK) return fail(c, st, "lbmc_set_closure: model is on another device or the image build failed");
@@ -857,7 +1039,7 @@ lbmc_status lbmc_set_closure_interval(lbmc_ctx *c, int every)
     if (every < 1 || every > 4096) return fail(c, LBMC_ERR_INVALID, "lbmc_set_closure_interval: interval %d not in [1, 4096]", every);
     if (every > 1 && !c->tcache) {
         HIP_TRY(c, hipSetDevice(c->desc.device), "hipSetDevice");
-        HIP_TRY(c, hipMalloc((void **)&c->tcache, sizeof(float) * (size_t)c->npad), "closure tau record");
+        HIP_TRY(c, dev_malloc((void **)&c->tcache, sizeof(float) * (size_t)c->npad), "closure tau record");
     }
     c->closure_every = every;
     c->tcache_valid = false;

@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "../../include/lbmc.h"
+#include "dispatch.hpp"
 #include "mlp.hpp"
 
 namespace lbmc {
@@ -356,7 +357,7 @@ lbmc_status ensure_partial(lbmc_mlp *m, int nw)
     if (nw <= m->pcap) return LBMC_OK;
     if (m->partial) MLP_HIP(m, hipFree(m->partial));
     m->partial = nullptr;
-    MLP_HIP(m, hipMalloc(&m->partial, (size_t)nw * MLP_PSTRIDE * sizeof(float)));
+    MLP_HIP(m, dev_malloc((void **)&m->partial, (size_t)nw * MLP_PSTRIDE * sizeof(float)));
     m->pcap = nw;
     return LBMC_OK;
 }
@@ -406,9 +407,9 @@ lbmc_status upload_data(lbmc_mlp *m, const float *feat, const float *target, lon
     m->feat = m->target = nullptr;
     m->order = nullptr;
     m->S = 0;
-    MLP_HIP(m, hipMalloc(&m->feat, (size_t)S * 7 * sizeof(float)));
-    MLP_HIP(m, hipMalloc(&m->target, (size_t)S * sizeof(float)));
-    MLP_HIP(m, hipMalloc(&m->order, (size_t)S * sizeof(int)));
+    MLP_HIP(m, dev_malloc((void **)&m->feat, (size_t)S * 7 * sizeof(float)));
+    MLP_HIP(m, dev_malloc((void **)&m->target, (size_t)S * sizeof(float)));
+    MLP_HIP(m, dev_malloc((void **)&m->order, (size_t)S * sizeof(int)));
     MLP_HIP(m, hipMemcpy(m->feat, feat, (size_t)S * 7 * sizeof(float), hipMemcpyHostToDevice));
     if (target) MLP_HIP(m, hipMemcpy(m->target, target, (size_t)S * sizeof(float), hipMemcpyHostToDevice));
     else MLP_HIP(m, hipMemset(m->target, 0, (size_t)S * sizeof(float)));
@@ -464,12 +465,12 @@ lbmc_status lbmc_mlp_create(int device, const float *params, const lbmc_mlp_scal
     };
     chk(hipSetDevice(device), "hipSetDevice");
     chk(hipStreamCreate(&m->stream), "hipStreamCreate");
-    chk(hipMalloc(&m->params, MLP_NPARAM * sizeof(float)), "hipMalloc");
-    chk(hipMalloc(&m->m1, MLP_NPARAM * sizeof(float)), "hipMalloc");
-    chk(hipMalloc(&m->m2, MLP_NPARAM * sizeof(float)), "hipMalloc");
-    chk(hipMalloc(&m->grad, MLP_NPARAM * sizeof(float)), "hipMalloc");
-    chk(hipMalloc(&m->img, sizeof(MlpImage)), "hipMalloc");
-    chk(hipMalloc(&m->lossacc, sizeof(double)), "hipMalloc");
+    chk(dev_malloc((void **)&m->params, MLP_NPARAM * sizeof(float)), "hipMalloc");
+    chk(dev_malloc((void **)&m->m1, MLP_NPARAM * sizeof(float)), "hipMalloc");
+    chk(dev_malloc((void **)&m->m2, MLP_NPARAM * sizeof(float)), "hipMalloc");
+    chk(dev_malloc((void **)&m->grad, MLP_NPARAM * sizeof(float)), "hipMalloc");
+    chk(dev_malloc((void **)&m->img, sizeof(MlpImage)), "hipMalloc");
+    chk(dev_malloc((void **)&m->lossacc, sizeof(double)), "hipMalloc");
     if (st == LBMC_OK) {
         chk(hipMemcpy(m->params, params, MLP_NPARAM * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
         chk(hipMemset(m->m1, 0, MLP_NPARAM * sizeof(float)), "hipMemset");
@@ -539,8 +540,8 @@ lbmc_status lbmc_mlp_forward(lbmc_mlp *m, const float *feat, long long S, float 
     if (S > (1LL << 31) / 8) return mfail(m, LBMC_ERR_INVALID, "lbmc_mlp_forward: too many samples");
     MLP_HIP(m, hipSetDevice(m->device));
     float *dx = nullptr, *dy = nullptr;
-    MLP_HIP(m, hipMalloc(&dx, (size_t)S * 7 * sizeof(float)));
-    hipError_t e = hipMalloc(&dy, (size_t)S * sizeof(float));
+    MLP_HIP(m, dev_malloc((void **)&dx, (size_t)S * 7 * sizeof(float)));
+    hipError_t e = dev_malloc((void **)&dy, (size_t)S * sizeof(float));
     if (e == hipSuccess) e = hipMemcpyAsync(dx, feat, (size_t)S * 7 * sizeof(float), hipMemcpyHostToDevice, m->stream);
     if (e == hipSuccess) {
         if (m->eval_fp16)

@@ -34,10 +34,11 @@ namespace lbmc {
 // the node's pulled populations as stored (f_i, or g_i = f_i - w_i for the
 // shifted formats) converted to the compute type; on return v[] holds the
 // post-collision values in the same form, ready to be written back to the
-// same slots.  Stores rho/u when the call asks for it.
+// same slots.  desc is the descriptor of the node's class (0: plain fluid);
+// stores rho/u when asked (store).
 template <class L, class St, int FAM, bool GUO, bool SMAG, bool MFIX>
-__device__ __forceinline__ void node_update(const StepArgs<typename St::C> &a, int n,
-                                            typename St::C (&v)[L::Q])
+__device__ __forceinline__ void node_update_as(const StepArgs<typename St::C> &a, int n, uint16_t desc, bool store,
+                                               typename St::C (&v)[L::Q])
 {
     using C = typename St::C;
     constexpr int Q = L::Q;
@@ -48,9 +49,8 @@ __device__ __forceinline__ void node_update(const StepArgs<typename St::C> &a, i
     // FP32 compute: plain fluid nodes of the BGK family take the regrouped
     // update (fast_bgk.hpp); everything else follows the reference's order.
     constexpr bool FAST = std::is_same<C, float>::value;
-    const unsigned m = a.all_fluid ? 0u : ldg(a.mask + n);
     if constexpr (FAST && FAM == 0) {
-        if (m == 0) {
+        if (desc == 0) {
             C F[3] = {C(0), C(0), C(0)};
             if constexpr (GUO) {
                 sfor<0, D>([&](auto dd) {
@@ -60,7 +60,7 @@ __device__ __forceinline__ void node_update(const StepArgs<typename St::C> &a, i
             }
             C rho, u[3];
             fluid_bgk_fast<L, St::shifted, GUO, SMAG>(v, a.tau, a.c_smag, F, rho, u);
-            if (a.store) {
+            if (store) {
                 sfor<0, D>([&](auto dd) {
                     constexpr int d = decltype(dd)::value;
                     stg(a.u[d] + n, u[d]);
@@ -108,8 +108,6 @@ __device__ __forceinline__ void node_update(const StepArgs<typename St::C> &a, i
     }
 
     // ---- node class
-    const uint16_t desc = m ? ldg(a.cls + m) : (uint16_t)0;
-
     bool stored_done = false;
     if (desc & CLS_SOLID) {
         // bounceback, collision.cu:423-443
@@ -289,13 +287,30 @@ __device__ __forceinline__ void node_update(const StepArgs<typename St::C> &a, i
             else v[i] = f[i];
         });
     }
-    if (a.store) {
+    if (store) {
         sfor<0, D>([&](auto dd) {
             constexpr int d = decltype(dd)::value;
             stg(a.u[d] + n, u[d]);
         });
         stg(a.rho + n, rho);
     }
+}
+
+// Descriptor of a node's class; class 0 is plain fluid, every other class has
+// a nonzero descriptor.
+template <class C>
+__device__ __forceinline__ uint16_t node_class(const StepArgs<C> &a, int n)
+{
+    const unsigned m = a.all_fluid ? 0u : ldg(a.mask + n);
+    return m ? ldg(a.cls + m) : (uint16_t)0;
+}
+
+// the same with the node's class from the mask and the call's store flag
+template <class L, class St, int FAM, bool GUO, bool SMAG, bool MFIX>
+__device__ __forceinline__ void node_update(const StepArgs<typename St::C> &a, int n,
+                                            typename St::C (&v)[L::Q])
+{
+    node_update_as<L, St, FAM, GUO, SMAG, MFIX>(a, n, node_class(a, n), a.store != 0, v);
 }
 
 // n / d for 0 <= n < 2^31 with the magic pair (m, l) of d

@@ -1,0 +1,12 @@
+// D2Q9 tile kernels with StFP16S population storage.
+#include "tile_launch.hpp"
+
+namespace lbmc {
+
+hipError_t launch_tile_fp16s(const KernelKey &k, int size, const StepArgs<float> &a, const TilePass &p, int tiles,
+                          hipStream_t s)
+{
+    return launch_tile_st<StFP16S>(k, size, a, p, tiles, s);
+}
+
+}  // namespace lbmc
