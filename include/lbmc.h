@@ -133,7 +133,8 @@ lbmc_status lbmc_step(lbmc_ctx *ctx, long long t, int store_macros);
 
 /* nsteps calls with t = t0 .. t0+nsteps-1; macros are stored on the calls
  * where (t+1) % store_every == 0 (store_every <= 0: never).  Lattices whose
- * calls the library runs several at a time (D2Q9 without sf boundaries) hold
+ * calls the library runs several at a time (D2Q9 without sf boundaries; D3Q15
+ * BGK lattices of fluid and solid nodes with FP64 or FP32 storage) hold
  * a second population array from lbmc_set_fields on, taken only while half
  * of the device's memory stays free and given back when a later allocation
  * of the library does not fit; the results do not depend on it. */

@@ -62,12 +62,14 @@ struct lbmc_ctx {
     float *tcache = nullptr;
     bool tcache_valid = false;
 
-    // passes of several calls (tile_kernel.hpp): tile shape, and the second
+    // passes of several calls (tile_kernel.hpp, march_kernel.hpp): tile shape, and the second
     // population buffer that they write to (null: one call per launch).
     // pass_mu: held while launches that use f2 are issued, and by another
     // thread that takes f2 back when device memory runs out (dev_malloc)
     lbmc::TilePlan tile{};
     void *f2 = nullptr;
+    long long npad2 = 0;  // elements between f2's direction arrays
+    int march_cls = 0;  // node classes of a D3Q15 lattice's passes (MARCH_*)
     std::mutex pass_mu;
     bool has_macro = false;  // some node prescribes rho or u from the macro arrays
 

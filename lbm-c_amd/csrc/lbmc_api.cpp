@@ -196,28 +196,46 @@ void drop_passes(lbmc_ctx *c)
 }
 
 // Tiles of the passes over a lattice and their second population buffer:
-// D2Q9 lattices without sf nodes whose direction arrays 32-bit offsets
-// reach.  The buffer is taken only while half of the device's memory stays
+// lattices without sf nodes, D2Q9 ones whose direction arrays 32-bit offsets
+// reach, D3Q15 ones of fluid and solid nodes, BGK family, in 32 and 64 bits,
+// whose planes they reach.  The buffer is taken only while half of the device's memory stays
 // free, and given back when an allocation fails (dev_malloc), so that a
 // program's lattices fit as they would without it.
 void plan_passes(lbmc_ctx *c)
 {
     std::lock_guard<std::mutex> lock(c->pass_mu);
     TilePlan q;
-    if (c->D == 2 && !c->nsf && !c->offsets64) {
-        int ncu = 256;
-        (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->desc.device);
-        q = plan_tiles(c->L[0], c->L[1], (int)c->sbytes, std::max(1, ncu));
-        // test hook: LBMC_PASS=0 one call per launch, or "size,W,H,M" a tile shape
-        if (const char *env = getenv("LBMC_PASS")) {
-            int v[4] = {0, 0, 0, 0};
-            q = TilePlan{};
-            if (sscanf(env, "%d,%d,%d,%d", &v[0], &v[1], &v[2], &v[3]) == 4 && v[0] >= 0 && v[0] <= 2 && v[3] >= 0 &&
-                v[3] < 32) {
-                const TileCapacity cap = tile_capacity(v[0], (int)c->sbytes);
-                q.on = (long long)v[1] * v[2] <= cap.threads * cap.per_thread &&
-                       tile_shape(c->L[0], c->L[1], v[0], v[1], v[2], v[3], q);
-            }
+    int ncu = 256;
+    (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->desc.device);
+    ncu = std::max(1, ncu);
+    const int slot = (int)c->sbytes;
+    // test hook: LBMC_PASS=0 one call per launch, "size,W,H,M" a tile shape
+    // of D2Q9 lattices, "W,H,nz" tiles and z ranges of D3Q15 ones
+    const char *env = getenv("LBMC_PASS");
+    int v[4] = {0, 0, 0, 0};
+    const int nv = env ? sscanf(env, "%d,%d,%d,%d", &v[0], &v[1], &v[2], &v[3]) : 0;
+    if (c->nsf) {
+        // the sf gather reads the state before every call
+    } else if (c->D == 2 && !c->offsets64) {
+        if (!env) {
+            q = plan_tiles(c->L[0], c->L[1], slot, ncu);
+        } else if (nv == 4 && v[0] >= 0 && v[0] <= 2 && v[3] < 32) {
+            const TileCapacity cap = tile_capacity(v[0], slot);
+            q.on = (long long)v[1] * v[2] <= cap.threads * cap.per_thread &&
+                   tile_shape(c->L[0], c->L[1], v[0], v[1], v[2], v[3], q);
+        }
+    } else if (c->D == 3 && c->key.family == 0 && slot >= 4 &&
+               (unsigned long long)c->L[0] * c->L[1] * slot < (1ULL << 31)) {
+        c->march_cls = c->all_fluid ? MARCH_FLUID : MARCH_SOLID;
+        bool plain = true;
+        for (int k = 1; k < c->ncls; k++) plain = plain && c->cls_host[k] == CLS_SOLID;
+        if (!plain) {
+            // boundary or porous nodes: one call per launch
+        } else if (!env) {
+            q = plan_march(c->L, slot, ncu);
+        } else if (nv == 3 && v[0] >= 3 && v[1] >= 3 && v[2] >= 1) {
+            q.on = (long long)v[0] * v[1] <= march_threads(slot);
+            march_shape(c->L, v[0], v[1], std::min(v[2], c->L[2]), q);
         }
     }
     if (!q.on) {
@@ -225,7 +243,7 @@ void plan_passes(lbmc_ctx *c)
         return;
     }
     if (!c->f2) {
-        const size_t bytes = c->sbytes * (size_t)c->Q * (size_t)c->npad;
+        const size_t bytes = c->sbytes * (size_t)c->Q * (size_t)c->npad2;
         size_t avail = 0, total = 0;
         if (hipMemGetInfo(&avail, &total) != hipSuccess || avail < bytes + total / 2 ||
             hipMalloc(&c->f2, bytes) != hipSuccess) {
@@ -279,6 +297,23 @@ hipError_t launch_pass(lbmc_ctx *c, long long t, int calls, unsigned store, bool
 {
     StepArgs<C> a;
     fill_args(c, a, t, 0);
+    if (c->D == 3) {
+        MarchPass p;
+        memset(&p, 0, sizeof(p));
+        march_geometry(c->tile, p);
+        p.src = src;
+        p.dst = dst;
+        p.store = store;
+        for (int d = 0; d < 3; d++) {
+            p.rs[d] = first ? a.s[d] : 1 % c->L[d];
+            p.ws[d] = last ? (int)((t + calls - 1) % c->L[d]) : 0;
+        }
+        p.rstride = src == c->f ? c->npad : c->npad2;
+        p.wstride = dst == c->f ? c->npad : c->npad2;
+        p.cls = c->march_cls;
+        if constexpr (sizeof(C) == 8) return launch_march_fp64(c->key, a, p, c->stream);
+        else return launch_march_fp32(c->key, a, p, c->stream);
+    }
     TilePass p;
     memset(&p, 0, sizeof(p));
     tile_geometry(c->tile, c->L, p);
@@ -304,11 +339,14 @@ hipError_t launch_pass(lbmc_ctx *c, long long t, int calls, unsigned store, bool
 }
 
 // len >= 2 calls from t: an even number of passes, so that the state ends in
-// the buffer it started in
+// the buffer it started in.  D2Q9 passes share the calls out evenly; D3Q15
+// passes take two each, and the last up to three calls run one by one.
 lbmc_status run_passes(lbmc_ctx *c, long long t, long long len, int store_every)
 {
     const int K = c->tile.M + 1;
-    const long long np = 2 * ((len + 2 * K - 1) / (2 * K));
+    const long long np = c->D == 2 ? 2 * ((len + 2 * K - 1) / (2 * K)) : 2 * (len / (2 * K));
+    long long rest = c->D == 2 ? 0 : len - K * np;
+    len -= rest;
     for (long long k = 0; k < np; k++) {
         const long long k0 = len * k / np, k1 = len * (k + 1) / np;
         unsigned store = 0;
@@ -321,6 +359,8 @@ lbmc_status run_passes(lbmc_ctx *c, long long t, long long len, int store_every)
                            : launch_pass<float>(c, t + k0, (int)(k1 - k0), store, k == 0, k + 1 == np, src, dst);
         if (e != hipSuccess) return hip_fail(c, e, "pass launch");
     }
+    for (t += len; rest > 0; rest--, t++)
+        if (lbmc_status st = launch_step(c, t, store_every > 0 && (t + 1) % store_every == 0)) return st;
     return LBMC_OK;
 }
 
@@ -470,6 +510,12 @@ lbmc_status lbmc_create(const lbmc_desc *desc, lbmc_ctx **out)
     for (int d = 0; d < 3; d++) c->L[d] = d < D ? desc->length[d] : 1;
     c->N = N;
     c->npad = (N + 63) / 64 * 64;
+    // the second buffer's direction arrays of D3Q15 a few cache lines apart:
+    // at 256^3 the starts of unpadded arrays are congruent in every L2 set and
+    // the side columns of the march passes miss (1.45 GB fetched per pass
+    // instead of 1.10; 234 us per call, 218 with the second buffer padded;
+    // padding both is 2 % better still, but costs one call per launch 2-3 %)
+    c->npad2 = c->npad + (D == 3 ? 96 : 0);
     c->storage = desc->storage;
     c->sbytes = desc->storage == LBMC_FP64 ? 8 : desc->storage == LBMC_FP32 ? 4 : 2;
     c->cbytes = desc->storage == LBMC_FP64 ? 8 : 4;

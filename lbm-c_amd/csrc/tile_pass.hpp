@@ -1,5 +1,6 @@
-// Arguments and planning of the passes that run several calls of a D2Q9
-// lattice at once (tile_kernel.hpp).
+// Arguments and planning of the passes that run several calls at once: tiles
+// of a D2Q9 lattice (tile_kernel.hpp), marching columns of a D3Q15 one
+// (march_kernel.hpp).
 #pragma once
 
 #include <algorithm>
@@ -26,12 +27,41 @@ struct TilePass {
     int s0[2];           // t mod L of the pass's first call (stochastic rounding)
 };
 
+// Node classes of a D3Q15 lattice's passes: plain fluid; fluid and solid.
+// Lattices with boundary or porous nodes have no passes: the node update with
+// every boundary condition needs 133-157 registers (768 threads per block),
+// and measured 0.5-1.0 of one call per launch.
+enum { MARCH_FLUID = 0, MARCH_SOLID = 1 };
+
+// Two calls of a D3Q15 lattice
+struct MarchPass {
+    const void *src;
+    void *dst;
+    long long rstride, wstride;  // elements between the direction arrays of src and dst
+    unsigned store;     // bit j: call j of the pass stores rho / u
+    int W, H, OW, OH;   // columns of a tile, owned columns
+    unsigned mw;        // magic pair of W
+    int lw;
+    int ntx;            // tiles along x, and their magic pair
+    unsigned mn;
+    int ln;
+    int tiles;          // tiles of a plane, and their magic pair
+    unsigned mt;
+    int lt;
+    int OZ;             // planes of a z range
+    int blocks;         // tiles * z ranges
+    int per_xcd;        // ceil(blocks / 8); the grid is 8 * per_xcd
+    int rs[3], ws[3];   // read and write shifts, mod L
+    int cls;            // MARCH_*
+};
+
 // Tiles of a lattice: the kernel's capacity (size, tile_capacity), the margin
 // M = calls of a pass - 1 and the tile shape.
 struct TilePlan {
     bool on = false;
     int size = 0, W = 0, H = 0, M = 0, OW = 0, OH = 0, ntx = 0, nty = 0;
-    double us = 0;  // estimated time per call
+    int OZ = 0, nz = 0;  // D3Q15: planes per z range, z ranges
+    double us = 0;       // estimated time per call
 };
 
 // Kernel capacities: threads per block and nodes per thread.  Sizes 0 and 1
@@ -129,6 +159,112 @@ inline void tile_geometry(const TilePlan &q, const int *L, TilePass &p)
     p.lt = dt.l;
     p.xoff = (q.M + L[0] - 1) / L[0] * L[0];
     p.yoff = (q.M + L[1] - 1) / L[1] * L[1];
+}
+
+// Threads per block of the march kernels, by the registers that a column
+// needs: 128 are available at 1024 threads (102-125 used), 256 at 512 (202-245
+// in 64 bits).
+constexpr int march_threads(int slot_bytes) { return slot_bytes == 8 ? 512 : 1024; }
+
+inline void march_shape(const int *L, int W, int H, int nz, TilePlan &q)
+{
+    q.M = 1;
+    q.ntx = (L[0] + W - 3) / (W - 2);
+    q.nty = (L[1] + H - 3) / (H - 2);
+    q.OW = (L[0] + q.ntx - 1) / q.ntx;
+    q.OH = (L[1] + q.nty - 1) / q.nty;
+    q.W = q.OW + 2;
+    q.H = q.OH + 2;
+    q.OZ = (L[2] + nz - 1) / nz;
+    q.nz = (L[2] + q.OZ - 1) / q.OZ;
+}
+
+// Estimated time per call (us) of the march passes of a plan: 2 us per launch
+// and an iteration (one plane of every resident block) of b + c * MB, MB the
+// traffic of the resident blocks with e bytes of partial lines at the ends of
+// every tile row.  b, c and e fitted to 260 shapes on 11 lattices (within 4-10
+// % of the measured times; the chosen shape 0-4 % from the best), apart for
+// lattices whose two buffers fit the 256 MB last-level cache.
+inline double march_estimate(const TilePlan &q, const int *L, int slot_bytes, int ncu)
+{
+    const double s = slot_bytes;
+    const bool cached = 2.0 * 15 * s * L[0] * L[1] * L[2] <= 260e6;
+    const double e = slot_bytes == 8 ? (cached ? 64 : 96) : (cached ? 160 : 64);
+    const double b = slot_bytes == 8 ? (cached ? 4.5 : 3.3) : (cached ? 2.7 : 0.6);
+    const double c = cached ? 0.015 : slot_bytes == 8 ? 0.075 : 0.135;
+    const bool aligned = q.OW * slot_bytes % 128 == 0 && L[0] * slot_bytes % 128 == 0;
+    const double bytes = 15 * (q.H * (q.W * s + e) + q.OH * (q.OW * s + (aligned ? 0 : e)));
+    const double blocks = (double)q.ntx * q.nty * q.nz;
+    const double rounds = (double)((long long)((blocks + ncu - 1) / ncu));
+    const double mb = (blocks < ncu ? blocks : ncu) * bytes * 1e-6;
+    return (2.0 + rounds * (q.OZ + 2) * (b + c * mb)) / 2;
+}
+
+// One call per launch: 2 us, then 6 TB/s where the populations stay in the
+// 256 MB last-level cache, 5.6 TB/s from HBM.
+inline double march_step_estimate(double nodes, int slot_bytes)
+{
+    const double bytes = nodes * 15 * slot_bytes;
+    return 2.0 + 2 * bytes / (bytes <= 256e6 ? 6e6 : 5.6e6);
+}
+
+// The plan with the smallest estimate, or none where one call per launch is
+// estimated within 5 % of it (lattices below ~6e5 nodes: too few columns for
+// 256 CUs).
+// Measured, us per call, one call per launch -> passes: FP32 BGK with
+// Smagorinsky, all fluid, 256^3 357 -> 230, 512^3 3005 -> 1774, 128^3 39.1 ->
+// 26, 131 x 97 x 75 21.6 -> 13.5; forced duct with solid walls 256^3 373 ->
+// 273, 131 x 97 x 75 23.9 -> 17.6; FP64 256^3 771 -> 551, 200 x 150 x 100
+// 137 -> 109; 64^3 6.2 against 8.3 in passes (not planned).  FP64 lattices
+// that fit the last-level cache once but not twice stay with one call per
+// launch (128^3: 74.6 against 75.0).  16-bit lattices have no passes: 256^3
+// 192 us against 221, bound by the arithmetic that a pass repeats at the sides.
+inline TilePlan plan_march(const int *L, int slot_bytes, int ncu)
+{
+    TilePlan best;
+    if (slot_bytes < 4) return best;
+    const double nodes = (double)L[0] * L[1] * L[2], bytes = nodes * 15 * slot_bytes;
+    if (slot_bytes == 8 && bytes > 128e6 && bytes <= 256e6) return best;
+    best.us = 0.95 * march_step_estimate(nodes, slot_bytes);
+    const int T = march_threads(slot_bytes);
+    for (int k = 1; k <= 64 && k <= L[0]; k++) {
+        const int W = (L[0] + k - 1) / k + 2, H = std::min(T / W, L[1] + 2);
+        if (W < 18 && k > 1) break;
+        if (H < 3) continue;
+        const int tiles = ((L[0] + W - 3) / (W - 2)) * ((L[1] + H - 3) / (H - 2));
+        for (int r = 1; r <= 4; r++) {
+            // the most z ranges that r rounds of blocks hold
+            const int nz = std::max(1, std::min((r * ncu) / tiles, L[2]));
+            TilePlan q;
+            march_shape(L, W, H, nz, q);
+            q.us = march_estimate(q, L, slot_bytes, ncu);
+            if (q.us < best.us) {
+                best = q;
+                best.on = true;
+            }
+        }
+    }
+    return best;
+}
+
+inline void march_geometry(const TilePlan &q, MarchPass &p)
+{
+    p.W = q.W;
+    p.H = q.H;
+    p.OW = q.OW;
+    p.OH = q.OH;
+    p.ntx = q.ntx;
+    p.tiles = q.ntx * q.nty;
+    const FastDiv dw = make_fastdiv(q.W), dn = make_fastdiv(q.ntx), dt = make_fastdiv(p.tiles);
+    p.mw = dw.m;
+    p.lw = dw.l;
+    p.mn = dn.m;
+    p.ln = dn.l;
+    p.mt = dt.m;
+    p.lt = dt.l;
+    p.OZ = q.OZ;
+    p.blocks = p.tiles * q.nz;
+    p.per_xcd = (p.blocks + 7) / 8;
 }
 
 }  // namespace lbmc

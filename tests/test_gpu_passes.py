@@ -1,6 +1,7 @@
-"""Passes of several calls (lbmc_run on D2Q9 lattices) against one call per
+"""Passes of several calls (lbmc_run) against one call per
 launch, bit for bit: the same node updates in another order of memory traffic.
-LBMC_PASS=0 keeps one call per launch, "size,W,H,M" forces a tile shape."""
+LBMC_PASS=0 keeps one call per launch; "size,W,H,M" (D2Q9) and "W,H,nz"
+(D3Q15) force a tile shape."""
 import numpy as np
 import pytest
 
@@ -54,5 +55,62 @@ def test_long_time_index_and_late_start(monkeypatch):
     case = cases.channel_d2q9(37, 21)
     want = _run(monkeypatch, case, 0, "0", 3, t0=2 ** 31 + 5)
     got = _run(monkeypatch, case, 0, None, 3, t0=2 ** 31 + 5)
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)
+
+
+def _duct(forcing):
+    """A box with solid walls on four sides and a solid block inside."""
+    L = (37, 22, 11)
+    c = cases.turbulence_d3q15(1, forcing=False)
+    n = L[0] * L[1] * L[2]
+    rng = np.random.default_rng(5)
+    geo = np.zeros((L[2], L[1], L[0]))
+    geo[0] = geo[-1] = 1
+    geo[:, 0] = geo[:, -1] = 1
+    geo[4:6, 8:12, 10:17] = 1
+    force = [np.full(n, 1e-5), 1e-6 * rng.standard_normal(n), np.zeros(n)] if forcing else None
+    return dict(c, name=f"duct_d3q15_g{int(forcing)}",
+                desc=dict(c["desc"], length=L, forcing=forcing, c_smag=0.1 if forcing else 0.0),
+                fields=dict(geometry=geo.reshape(-1), force=force),
+                init=("equilibrium", 1 + 0.01 * rng.standard_normal(n), cases.random_velocity(rng, (L[2], L[1], L[0]), 0.02)))
+
+
+D3_CASES = [
+    cases.turbulence_d3q15(12),
+    cases.turbulence_d3q15(35, c_smag=0.0),
+    cases.turbulence_d3q15(13, forcing=True),
+    _duct(False),
+    _duct(True),
+    cases.turbulence_d3q15(12, collision=cases.MRT),  # no passes: the hook changes nothing
+    cases.faces_d3q15(),                              # boundary nodes: no passes either
+]
+
+
+@pytest.mark.parametrize("storage", [0, 1, 2], ids=["f64", "f32", "f16s"])
+@pytest.mark.parametrize("case", D3_CASES, ids=lambda c: c["name"])
+def test_march_matches_one_call_per_launch(monkeypatch, case, storage):
+    for store_every in (0, 1, 5):
+        want = _run(monkeypatch, case, storage, "0", store_every)
+        # whole rows and several z ranges, small uneven tiles, the smallest
+        # tile with single-plane ranges, a tile larger than the lattice
+        for shape in ("37,13,3", "9,7,2", "3,3,64", "64,8,1"):
+            got = _run(monkeypatch, case, storage, shape, store_every)
+            for a, b in zip(got, want):
+                assert np.array_equal(a, b), (shape, store_every)
+
+
+@pytest.mark.parametrize("storage", [0, 1], ids=["f64", "f32"])
+def test_march_planned_shape(monkeypatch, storage):
+    # large enough for the planner to choose passes by itself
+    case = cases.turbulence_d3q15(1)
+    L = (131, 96, 75)
+    n = L[0] * L[1] * L[2]
+    rng = np.random.default_rng(8)
+    case = dict(case, desc=dict(case["desc"], length=L), fields=dict(geometry=np.zeros(n)),
+                init=("equilibrium", 1 + 0.01 * rng.standard_normal(n),
+                      cases.random_velocity(rng, (L[2], L[1], L[0]), 0.02)))
+    want = _run(monkeypatch, case, storage, "0", 5)
+    got = _run(monkeypatch, case, storage, None, 5)
     for a, b in zip(got, want):
         assert np.array_equal(a, b)
