@@ -3,10 +3,10 @@
 // lbmc_mlp_*).
 //
 // One training step over a minibatch of B samples:
-//   1. mlp_train_kernel: one wave per 64 samples computes the forward pass,
-//      the backward pass and its partial gradient (per-wave record);
-//   2. mlp_update_kernel: one thread per parameter sums the records in wave
-//      order (deterministic) and applies Adam to the FP32 master weights;
+//   1. mlp_train_kernel: one block per 64 samples computes the forward pass,
+//      the backward pass and its partial gradient (a record per block);
+//   2. mlp_update_kernel: sums the records in block order (deterministic)
+//      and applies Adam to the FP32 master weights;
 //   3. mlp_image_kernel: rebuilds the operand images (bf16 for training,
 //      fp16 for evaluation) from the master weights.
 // The loss is the mean squared error over the minibatch.
@@ -139,64 +139,71 @@ __global__ __launch_bounds__(256) void mlp_forward_kernel(const MlpImage *img, c
     if (valid) y[i] = out;
 }
 
-// Per-wave LDS of the training kernel: matrices with the sample index
-// contiguous (rows padded to 72 entries), for the products that contract
-// over samples.
+// LDS of the training kernel: matrices with the sample index contiguous
+// (rows padded to 72 entries), for the products that contract over samples.
 struct alignas(16) MlpTrainLds {
     __bf16 a1[64][72];   // a1[k][n]
+    __bf16 a2[64][72];   // a2[i][n]
     __bf16 dz2[64][72];  // bf16 dL/dz2 [i][n]
     __bf16 dz1[64][72];  // bf16 dL/dz1 [i][n]
     __bf16 xt[16][72];   // inputs [f][n], rows 8..15 zero
+    float dzf[64][68];   // dL/dz2 [i][n] before rounding
     mlp_v8b xb[64];
     float tb[64];        // targets
     float sb[64];        // 1/B for samples in the batch, 0 for padding lanes
+    float dy[64], d2[64];  // dL/dy and (y - t)^2 per sample
 };
 
-// Forward and backward pass of 64 samples per block (one wave): writes the
-// wave's gradient of L = (1/B) sum (y - t)^2 and its sum of (y - t)^2.
-__global__ __launch_bounds__(64) void mlp_train_kernel(const MlpImage *img, const float *feat, const float *target,
-                                                       const int *order, long long first, int count, float invB,
-                                                       float *partial)
+// Forward and backward pass of 64 samples per block: writes the block's
+// gradient of L = (1/B) sum (y - t)^2 and its sum of (y - t)^2.
+//
+// Four waves: wave T takes the tile of samples 16 T .. 16 T + 15 through the
+// network, then the rows 16 T .. 16 T + 15 of the products and sums over the
+// 64 samples.  A minibatch of 16384 is 256 blocks, one per CU, so the time is
+// one block's chain of dependent products; one wave per block took the four
+// tiles one after the other, 19 us, four waves 11 us.  The sums run over the
+// tiles in the same order as that chain: same bits.
+__global__ __launch_bounds__(256) void mlp_train_kernel(const MlpImage *img, const float *feat, const float *target,
+                                                        const int *order, long long first, int count, float invB,
+                                                        float *partial)
 {
     __shared__ MlpTrainLds s;
     const MlpInfer &w = img->inf;
-    const int l = (int)threadIdx.x, g = l >> 4, r = l & 15;
-    const int i = (int)blockIdx.x * 64 + l;
-    const bool valid = i < count;
-    float f[7] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    float t = 0.f;
-    if (valid) {
-        const long long id = order ? (long long)order[first + i] : first + i;
-        for (int k = 0; k < 7; k++) f[k] = feat[id * 7 + k];
-        t = target[id];
+    const int T = (int)threadIdx.x >> 6;
+    const int l = (int)threadIdx.x & 63, g = l >> 4, r = l & 15;
+    if (g == 0) {
+        const int n = 16 * T + r;
+        const int i = (int)blockIdx.x * 64 + n;
+        const bool valid = i < count;
+        float f[7] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        float t = 0.f;
+        if (valid) {
+            const long long id = order ? (long long)order[first + i] : first + i;
+            for (int k = 0; k < 7; k++) f[k] = feat[id * 7 + k];
+            t = target[id];
+        }
+        mlp_v8b xin = mlp_input(w.sc, f);
+        if (!valid) {
+            for (int k = 0; k < 8; k++) xin[k] = (__bf16)0.f;
+        }
+        s.xb[n] = xin;
+        s.tb[n] = t;
+        s.sb[n] = valid ? invB : 0.f;
+        for (int k = 0; k < 8; k++) s.xt[k][n] = xin[k];
+        for (int k = 8; k < 16; k++) s.xt[k][n] = (__bf16)0.f;
     }
-    mlp_v8b xin = mlp_input(w.sc, f);
-    if (!valid) {
-        for (int k = 0; k < 8; k++) xin[k] = (__bf16)0.f;
-    }
-    s.xb[l] = xin;
-    s.tb[l] = t;
-    s.sb[l] = valid ? invB : 0.f;
-    for (int k = 0; k < 8; k++) s.xt[k][l] = xin[k];
-    for (int k = 8; k < 16; k++) s.xt[k][l] = (__bf16)0.f;
-    wave_sync();
+    __syncthreads();
 
     const mlp_v4f zero = {0.f, 0.f, 0.f, 0.f};
-    const float b3 = w.sc.b3;
-    float s2[4][4], s3[4][4];
-    for (int h = 0; h < 4; h++)
-        for (int j = 0; j < 4; j++) s2[h][j] = s3[h][j] = 0.f;
-    float loss = 0.f, gb3 = 0.f;
-#pragma unroll
-    for (int T = 0; T < 4; T++) {
+    {
         MlpTile o;
         mlp_tile_forward<true>(w, s.xb, T, l, o);
         const int n = 16 * T + r;
-        const float d = (o.y + b3) - s.tb[n];
+        const float d = (o.y + w.sc.b3) - s.tb[n];
         const float dy = 2.f * d * s.sb[n];
-        if (g == T) {
-            loss += s.sb[n] > 0.f ? d * d : 0.f;
-            gb3 += dy;
+        if (g == 0) {
+            s.d2[n] = s.sb[n] > 0.f ? d * d : 0.f;
+            s.dy[n] = dy;
         }
         mlp_v8b dzop[2];
 #pragma unroll
@@ -205,11 +212,11 @@ __global__ __launch_bounds__(64) void mlp_train_kernel(const MlpImage *img, cons
             for (int j = 0; j < 4; j++) {
                 const int row = 16 * h + 4 * g + j;
                 const float dz = img->w3d[h][l][j] * dy * gelu_grad(o.z2[h][j]);
-                s2[h][j] += dz;
-                s3[h][j] += (float)o.a2[h >> 1][(h & 1) * 4 + j] * dy;
+                s.dzf[row][n] = dz;
                 const __bf16 q = (__bf16)dz;
                 dzop[h >> 1][(h & 1) * 4 + j] = q;
                 s.dz2[row][n] = q;
+                s.a2[row][n] = o.a2[h >> 1][(h & 1) * 4 + j];
                 s.a1[row][n] = o.a1[h >> 1][(h & 1) * 4 + j];
             }
         }
@@ -221,69 +228,74 @@ __global__ __launch_bounds__(64) void mlp_train_kernel(const MlpImage *img, cons
             for (int j = 0; j < 4; j++) s.dz1[16 * h + 4 * g + j][n] = (__bf16)(da[j] * gelu_grad(o.z1[h][j]));
         }
     }
-    wave_sync();
+    __syncthreads();
 
     float *P = partial + (size_t)blockIdx.x * MLP_PSTRIDE;
     // dL/dW2 = dz2 a1^T and dL/dW1 = dz1 x^T: contractions over the 64 samples
 #pragma unroll
-    for (int hi = 0; hi < 4; hi++) {
-#pragma unroll
-        for (int hk = 0; hk < 4; hk++) {
-            mlp_v4f acc = zero;
-#pragma unroll
-            for (int c = 0; c < 2; c++) {
-                const mlp_v8b A = *(const mlp_v8b *)&s.dz2[16 * hi + r][32 * c + 8 * g];
-                const mlp_v8b B = *(const mlp_v8b *)&s.a1[16 * hk + r][32 * c + 8 * g];
-                acc = mfma_k32(A, B, acc);
-            }
-            for (int j = 0; j < 4; j++) P[MLP_W2 + (16 * hi + 4 * g + j) * 64 + 16 * hk + r] = acc[j];
-        }
-    }
-#pragma unroll
-    for (int hi = 0; hi < 4; hi++) {
+    for (int hk = 0; hk < 4; hk++) {
         mlp_v4f acc = zero;
 #pragma unroll
         for (int c = 0; c < 2; c++) {
-            const mlp_v8b A = *(const mlp_v8b *)&s.dz1[16 * hi + r][32 * c + 8 * g];
+            const mlp_v8b A = *(const mlp_v8b *)&s.dz2[16 * T + r][32 * c + 8 * g];
+            const mlp_v8b B = *(const mlp_v8b *)&s.a1[16 * hk + r][32 * c + 8 * g];
+            acc = mfma_k32(A, B, acc);
+        }
+        for (int j = 0; j < 4; j++) P[MLP_W2 + (16 * T + 4 * g + j) * 64 + 16 * hk + r] = acc[j];
+    }
+    {
+        mlp_v4f acc = zero;
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const mlp_v8b A = *(const mlp_v8b *)&s.dz1[16 * T + r][32 * c + 8 * g];
             const mlp_v8b B = *(const mlp_v8b *)&s.xt[r][32 * c + 8 * g];
             acc = mfma_k32(A, B, acc);
         }
         if (r < 8) {
-            for (int j = 0; j < 4; j++) P[MLP_W1 + (16 * hi + 4 * g + j) * 8 + r] = acc[j];
+            for (int j = 0; j < 4; j++) P[MLP_W1 + (16 * T + 4 * g + j) * 8 + r] = acc[j];
         }
     }
-    // dL/db2 and dL/dw3: sums over the 16 sample columns of each lane row
+    // dL/db2 and dL/dw3: per sample column the four tiles in order, then the
+    // sum over the 16 columns
 #pragma unroll
-    for (int h = 0; h < 4; h++) {
+    for (int j = 0; j < 4; j++) {
+        const int row = 16 * T + 4 * g + j;
+        float v2 = 0.f, v3 = 0.f;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            float v2 = s2[h][j], v3 = s3[h][j];
-            for (int m = 1; m < 16; m <<= 1) {
-                v2 += __shfl_xor(v2, m, 64);
-                v3 += __shfl_xor(v3, m, 64);
-            }
-            if (r == 0) {
-                P[MLP_B2 + 16 * h + 4 * g + j] = v2;
-                P[MLP_W3 + 16 * h + 4 * g + j] = v3;
-            }
+        for (int t = 0; t < 4; t++) {
+            v2 += s.dzf[row][16 * t + r];
+            v3 += (float)s.a2[row][16 * t + r] * s.dy[16 * t + r];
+        }
+        for (int m = 1; m < 16; m <<= 1) {
+            v2 += __shfl_xor(v2, m, 64);
+            v3 += __shfl_xor(v3, m, 64);
+        }
+        if (r == 0) {
+            P[MLP_B2 + row] = v2;
+            P[MLP_W3 + row] = v3;
         }
     }
-    for (int m = 1; m < 64; m <<= 1) {
-        loss += __shfl_xor(loss, m, 64);
-        gb3 += __shfl_xor(gb3, m, 64);
-    }
-    if (l == 0) {
-        P[MLP_B3] = gb3;
-        P[MLP_NPARAM] = loss;
+    if (T == 0) {
+        float loss = 0.f, gb3 = 0.f;
+        loss += s.d2[l];
+        gb3 += s.dy[l];
+        for (int m = 1; m < 64; m <<= 1) {
+            loss += __shfl_xor(loss, m, 64);
+            gb3 += __shfl_xor(gb3, m, 64);
+        }
+        if (l == 0) {
+            P[MLP_B3] = gb3;
+            P[MLP_NPARAM] = loss;
+        }
     }
 }
 
-// Sums the per-wave records in wave order; optional Adam step on the master
+// Sums the blocks' records in their order; optional Adam step on the master
 // weights (beta1 0.9, beta2 0.999, eps 1e-8; bc1/bc2 the bias corrections).
 //
 // A block takes 64 parameters: its 16 waves load 256 records' rows of them
 // (256 bytes each) into LDS at once, with the next 256 records' loads in
-// flight meanwhile, and the first wave adds them up in wave order, a lane per
+// flight meanwhile, and the first wave adds them up in that order, a lane per
 // parameter.  The order of the sum fixes the result, so only the loads can
 // be spread out: one thread per parameter loading and adding in turn (19
 // blocks) took 57 us for a minibatch of 16384 (256 records, 4.9 MB), bound by
@@ -422,7 +434,7 @@ lbmc_status grad_pass(lbmc_mlp *m, const int *order, long long first, int count,
     const int nw = (count + 63) / 64;
     lbmc_status st = ensure_partial(m, nw);
     if (st != LBMC_OK) return st;
-    hipLaunchKernelGGL(mlp_train_kernel, dim3(nw), dim3(64), 0, m->stream, m->img, m->feat, m->target, order,
+    hipLaunchKernelGGL(mlp_train_kernel, dim3(nw), dim3(256), 0, m->stream, m->img, m->feat, m->target, order,
                        first, count, 1.f / (float)count, m->partial);
     MLP_HIP(m, hipGetLastError());
     float bc1 = 1.f, bc2 = 1.f;
