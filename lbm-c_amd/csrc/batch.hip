@@ -27,15 +27,20 @@
 // is captured once into a HIP graph and replayed for any t.  The launch
 // shape of the step kernel is chosen by lbmc_batch_autotune (timed
 // candidates).
+//
+// D2Q9 members in 32 and 64 bits that all hold a second population buffer go
+// in passes of several calls instead (batch_tile_kernel.hpp, pass_steps).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cstdarg>
 #include <cstdio>
+#include <mutex>
 #include <string>
 #include <vector>
 
 #include "batch_kernel.hpp"
+#include "batch_tile_kernel.hpp"
 #include "ctx.hpp"
 #include "dispatch.hpp"
 #include "node_index.hpp"
@@ -70,6 +75,14 @@ struct lbmc_batch {
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     int graph_steps = 0;
+    // passes of several calls (batch_tile_kernel.hpp): the members' tiles, plain
+    // members' first (members of one collision variant together, which share
+    // the instruction cache), and the calls of a pass
+    std::vector<TilePlan> plans;
+    std::vector<char> tile_closure;  // which members the lists below hold as closure members
+    int2 *tiles = nullptr;
+    int ntiles_plain = 0, ntiles_closure = 0, pass_calls = 0;
+    void *dpass = nullptr;  // BatchTileMember<C>[count]: call t0 of the run
     const lbmc_mlp *closure_model = nullptr;
     double closure_lo = 0, closure_hi = 0;
     int closure_fp16 = 0;  // the closure members' network with fp16 operands
@@ -292,6 +305,198 @@ lbmc_status build_chunks(lbmc_batch *b, int sub)
     return LBMC_OK;
 }
 
+// ---- passes of several calls (D2Q9 members in 32 or 64 bits that all hold a
+// second population buffer)
+
+// tiles of every member, all of them with the margin of one pass length
+lbmc_status build_tiles(lbmc_batch *b)
+{
+    std::vector<char> closure;
+    for (const lbmc_ctx *c : b->members) closure.push_back(c->key.closure ? 1 : 0);
+    if (b->tiles && closure == b->tile_closure) return LBMC_OK;
+    const int slot = (int)b->members[0]->sbytes;
+    const TileCapacity cap = tile_capacity(2, slot);
+    const int P = cap.threads * cap.per_thread;
+    double best = -1;
+    for (int M = 1; M <= 6; M++) {
+        std::vector<TilePlan> plans;
+        double work = 0;
+        for (const lbmc_ctx *c : b->members) {
+            TilePlan q;
+            double w = -1;
+            for (int W = 16; W <= 128; W *= 2) {
+                TilePlan t;
+                if (!tile_shape(c->L[0], c->L[1], 2, W, P / W, M, t)) continue;
+                const double tw = tile_work(t, slot);
+                if (w < 0 || tw < w) {
+                    w = tw;
+                    q = t;
+                }
+            }
+            work += w;
+            plans.push_back(q);
+        }
+        if (best < 0 || work < best) {
+            best = work;
+            b->plans.swap(plans);
+            b->pass_calls = M + 1;
+        }
+    }
+    std::vector<int2> tiles;
+    for (int cl = 0; cl < 2; cl++) {
+        for (int v = 0; v < 10; v++)
+            for (int k = 0; k < b->count; k++)
+                if (closure[(size_t)k] == cl && member_variant(b->members[(size_t)k]) == v)
+                    for (int t = 0; t < b->plans[(size_t)k].ntx * b->plans[(size_t)k].nty; t++)
+                        tiles.push_back(make_int2(k, t));
+        (cl ? b->ntiles_closure : b->ntiles_plain) = (int)tiles.size() - (cl ? b->ntiles_plain : 0);
+    }
+    if (b->tiles) B_HIP(b, hipFree(b->tiles));
+    b->tiles = nullptr;
+    B_HIP(b, dev_malloc((void **)&b->tiles, sizeof(int2) * tiles.size()));
+    B_HIP(b, hipMemcpy(b->tiles, tiles.data(), sizeof(int2) * tiles.size(), hipMemcpyHostToDevice));
+    const size_t msz = b->cdouble ? sizeof(BatchTileMember<double>) : sizeof(BatchTileMember<float>);
+    if (!b->dpass) B_HIP(b, dev_malloc(&b->dpass, msz * (size_t)b->count));
+    b->tile_closure = closure;
+    return LBMC_OK;
+}
+
+// Whether a run from call t0 can go in passes: every member with a second
+// buffer (their pass_mu held), and closure members on one schedule.  *eval0:
+// the closure members evaluate on the first call.
+bool can_pass(const lbmc_batch *b, long long t0, int store_every, int *every, bool *eval0)
+{
+    if (b->lattice != LBMC_D2Q9 || (b->storage != LBMC_FP64 && b->storage != LBMC_FP32)) return false;
+    *every = 0;
+    *eval0 = false;
+    int seen = 0, ev = 0;
+    for (const lbmc_ctx *c : b->members) {
+        if (!c->f2 || !c->tile.on || c->nsf || !c->fields_set || c->L[0] >= (1 << 30) || c->L[1] >= (1 << 30)) return false;
+        // every few calls alone: one call per launch in place moves less
+        if (c->has_macro && store_every > 0 && store_every < 4) return false;
+        if (!c->key.closure) continue;
+        if (*every && c->closure_every != *every) return false;
+        *every = c->closure_every;
+        seen++;
+        ev += (c->closure_every == 1 || !c->tcache_valid || t0 % c->closure_every == 0) ? 1 : 0;
+    }
+    if (ev != 0 && ev != seen) return false;
+    *eval0 = ev != 0;
+    return true;
+}
+
+template <class C>
+lbmc_status upload_pass_members(lbmc_batch *b, long long t0)
+{
+    std::vector<BatchTileMember<C>> hm((size_t)b->count);
+    for (int k = 0; k < b->count; k++) {
+        const lbmc_ctx *c = b->members[(size_t)k];
+        if (c->key.closure && (c->closure_model != b->closure_model || c->closure_lo != b->closure_lo ||
+                               c->closure_hi != b->closure_hi || c->key.closure_fp16 != b->closure_fp16))
+            return bfail(b, LBMC_ERR_UNSUPPORTED, "batch member %d: closure members must share one model, band and operand precision", k);
+        BatchTileMember<C> &m = hm[(size_t)k];
+        memset(&m, 0, sizeof(m));
+        fill_args(c, m.a, t0, 0);
+        tile_geometry(b->plans[(size_t)k], c->L, m.p);
+        m.p.src = c->f;
+        m.p.dst = c->f2;
+        m.variant = member_variant(c);
+    }
+    B_HIP(b, hipMemcpyAsync(b->dpass, hm.data(), sizeof(BatchTileMember<C>) * hm.size(), hipMemcpyHostToDevice,
+                            b->stream));
+    B_HIP(b, hipStreamSynchronize(b->stream));
+    return LBMC_OK;
+}
+
+// The run's calls in passes; the device members describe call t0.  Returns
+// through *odd_* which buffer the members' states are in.
+lbmc_status pass_steps(lbmc_batch *b, long long t0, int nsteps, int store_every, int every, bool eval0, int *odd_plain,
+                       int *odd_closure)
+{
+    auto stores = [&](int k) { return store_every > 0 && (t0 + k + 1) % store_every == 0; };
+    bool macro[2] = {false, false};
+    for (const lbmc_ctx *c : b->members) macro[c->key.closure ? 1 : 0] |= c->has_macro;
+    // calls k .. end - 1 of one kind of members; calls that store the macros
+    // of members with prescribed values run alone (lbmc_run)
+    auto passes = [&](bool closure, int k, int end, int *odd) -> lbmc_status {
+        const int2 *tiles = b->tiles + (closure ? b->ntiles_plain : 0);
+        const int ntiles = closure ? b->ntiles_closure : b->ntiles_plain;
+        const int begin = k;
+        while (k < end) {
+            int e = end;
+            if (macro[closure ? 1 : 0] && store_every > 0) {
+                e = k;
+                while (e < end && !stores(e)) e++;
+                if (e == k) e = k + 1;
+            }
+            const int np = (e - k + b->pass_calls - 1) / b->pass_calls, k0 = k;
+            for (int q = 0; q < np; q++) {
+                BatchPass bp{};
+                bp.offset = k0 + (int)((long long)(e - k0) * q / np);
+                bp.calls = k0 + (int)((long long)(e - k0) * (q + 1) / np) - bp.offset;
+                for (int j = 0; j < bp.calls; j++)
+                    if (stores(bp.offset + j)) bp.store |= 1u << j;
+                bp.first = bp.offset == begin;
+                bp.last = bp.offset + bp.calls == end;
+                bp.odd = *odd;
+                const hipError_t err = b->cdouble ? launch_batch_tiles_fp64(b->dpass, tiles, ntiles, bp, b->stream)
+                                                  : launch_batch_tiles_fp32(b->dpass, tiles, ntiles, bp, b->stream);
+                if (err != hipSuccess)
+                    return bfail(b, LBMC_ERR_DEVICE, "batch pass launch: %s", hipGetErrorString(err));
+                *odd ^= 1;
+            }
+            k = e;
+        }
+        return LBMC_OK;
+    };
+    if (b->ntiles_plain)
+        if (lbmc_status st = passes(false, 0, nsteps, odd_plain)) return st;
+    if (b->ntiles_closure)
+        for (int k = 0; k < nsteps;) {
+            if (k == 0 ? eval0 : true) {
+                BatchPass bp{};
+                bp.offset = k;
+                bp.store = stores(k) ? 1u : 0u;
+                bp.odd = *odd_closure;
+                const hipError_t err = launch_batch_call_fp32(b->dpass, b->cchunks, b->ncchunks, b->eval_grid, b->sub,
+                                                              b->mlp, every > 1, b->closure_fp16 != 0, bp, b->stream);
+                if (err != hipSuccess)
+                    return bfail(b, LBMC_ERR_DEVICE, "batch call launch: %s", hipGetErrorString(err));
+                k++;
+            }
+            // recorded tau up to the next call with t % every == 0
+            const int end = (int)std::min<long long>(nsteps, (t0 + k + every - 1) / every * every - t0);
+            if (end > k)
+                if (lbmc_status st = passes(true, k, end, odd_closure)) return st;
+            k = std::max(k, end);
+        }
+    return LBMC_OK;
+}
+
+// Runs (timed: between the batch's events) in passes; *done false: not
+// possible, nothing was run
+lbmc_status run_in_passes(lbmc_batch *b, long long t0, int nsteps, int store_every, bool timed, bool *done)
+{
+    *done = false;
+    std::vector<std::unique_lock<std::mutex>> locks;
+    for (lbmc_ctx *c : b->members) locks.emplace_back(c->pass_mu);
+    int every = 0;
+    bool eval0 = false;
+    if (nsteps <= 0 || !can_pass(b, t0, store_every, &every, &eval0)) return LBMC_OK;
+    if (lbmc_status st = build_tiles(b)) return st;
+    if (b->ntiles_closure && (!b->mlp || !b->cchunks)) return LBMC_OK;
+    *done = true;
+    if (lbmc_status st = b->cdouble ? upload_pass_members<double>(b, t0) : upload_pass_members<float>(b, t0)) return st;
+    if (timed) B_HIP(b, hipEventRecord(b->ev0, b->stream));
+    int odd[2] = {0, 0};
+    const lbmc_status st = pass_steps(b, t0, nsteps, store_every, every, eval0, &odd[0], &odd[1]);
+    if (timed && st == LBMC_OK) B_HIP(b, hipEventRecord(b->ev1, b->stream));
+    B_HIP(b, hipStreamSynchronize(b->stream));
+    for (lbmc_ctx *c : b->members)
+        if (odd[c->key.closure ? 1 : 0]) swap_populations(c);
+    return st;
+}
+
 // after calls were run: every closure member with an interval now holds the
 // record of its last evaluation
 void mark_records(lbmc_batch *b)
@@ -387,6 +592,8 @@ lbmc_status lbmc_batch_create(lbmc_ctx *const *members, int count, lbmc_batch **
     b->grid = (int)std::min<long long>(b->nchunks, 8LL * b->ncu);
     if (hipDeviceGetAttribute(&b->lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, b->device) != hipSuccess)
         b->lds_cu = 0;
+    if (b->lattice == LBMC_D2Q9 && (b->storage == LBMC_FP64 || b->storage == LBMC_FP32))
+        if (lbmc_status st = build_tiles(b)) return bail(st);
     *out = b;
     return LBMC_OK;
 }
@@ -402,6 +609,8 @@ lbmc_status lbmc_batch_destroy(lbmc_batch *b)
     if (b->chunks) (void)hipFree(b->chunks);
     if (b->cchunks) (void)hipFree(b->cchunks);
     if (b->any_eval) (void)hipFree(b->any_eval);
+    if (b->tiles) (void)hipFree(b->tiles);
+    if (b->dpass) (void)hipFree(b->dpass);
     if (b->ev0) (void)hipEventDestroy(b->ev0);
     if (b->ev1) (void)hipEventDestroy(b->ev1);
     if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -414,8 +623,10 @@ lbmc_status lbmc_batch_run(lbmc_batch *b, long long t0, int nsteps, int store_ev
     if (!b || nsteps < 0 || t0 < 0) return bfail(b, LBMC_ERR_INVALID, "lbmc_batch_run: bad argument");
     B_HIP(b, hipSetDevice(b->device));
     lbmc_status st = sync_members(b);
-    if (st == LBMC_OK) st = upload(b, t0, store_every);
-    if (st == LBMC_OK) st = batch_steps(b, t0, nsteps);
+    bool done = false;
+    if (st == LBMC_OK) st = run_in_passes(b, t0, nsteps, store_every, false, &done);
+    if (st == LBMC_OK && !done) st = upload(b, t0, store_every);
+    if (st == LBMC_OK && !done) st = batch_steps(b, t0, nsteps);
     if (st != LBMC_OK) return st;
     if (nsteps > 0) mark_records(b);
     B_HIP(b, hipStreamSynchronize(b->stream));
@@ -427,13 +638,17 @@ lbmc_status lbmc_batch_time_steps(lbmc_batch *b, long long t0, int nsteps, int s
     if (!b || nsteps <= 0 || t0 < 0 || !ms) return bfail(b, LBMC_ERR_INVALID, "lbmc_batch_time_steps: bad argument");
     B_HIP(b, hipSetDevice(b->device));
     lbmc_status st = sync_members(b);
-    if (st == LBMC_OK) st = upload(b, t0, store_every);  // outside the timed region
+    bool done = false;
+    if (st == LBMC_OK) st = run_in_passes(b, t0, nsteps, store_every, true, &done);
+    if (st == LBMC_OK && !done) st = upload(b, t0, store_every);  // outside the timed region
     if (st != LBMC_OK) return st;
-    B_HIP(b, hipEventRecord(b->ev0, b->stream));
-    st = batch_steps(b, t0, nsteps);
-    if (st != LBMC_OK) return st;
+    if (!done) {
+        B_HIP(b, hipEventRecord(b->ev0, b->stream));
+        st = batch_steps(b, t0, nsteps);
+        if (st != LBMC_OK) return st;
+        B_HIP(b, hipEventRecord(b->ev1, b->stream));
+    }
     mark_records(b);
-    B_HIP(b, hipEventRecord(b->ev1, b->stream));
     B_HIP(b, hipEventSynchronize(b->ev1));
     B_HIP(b, hipEventElapsedTime(ms, b->ev0, b->ev1));
     return LBMC_OK;

@@ -127,8 +127,8 @@ __global__ __launch_bounds__(kBlock) void batch_step_kernel(const BatchMember<ty
                     // between evaluations: the recorded tau, no network
                     float v[L::Q];
                     gather_node<L, St, false>(a, n0, dd, v);
-                    if (variant == 9) closure_reuse_node<L, St, true>(a, n0, v);
-                    else closure_reuse_node<L, St, false>(a, n0, v);
+                    if (variant == 9) closure_reuse_node<L, St, true>(a, n0, node_class(a, n0), a.store != 0, v);
+                    else closure_reuse_node<L, St, false>(a, n0, node_class(a, n0), a.store != 0, v);
                     scatter_node<L, St, false>(a, n0, dd, v);
                     continue;
                 }
@@ -177,11 +177,11 @@ __global__ __launch_bounds__(kBlock, 4) void batch_eval_kernel(const BatchMember
             float v[L::Q];
             gather_node<L, St, false>(a, n, dd, v);
             if (a.tmode == 1) {
-                if (variant == 9) closure_update<L, St, true, true, H>(a, n, live, v, w, xw);
-                else closure_update<L, St, false, true, H>(a, n, live, v, w, xw);
+                if (variant == 9) closure_update<L, St, true, true, H>(a, n, live, a.store != 0, v, w, xw);
+                else closure_update<L, St, false, true, H>(a, n, live, a.store != 0, v, w, xw);
             } else {
-                if (variant == 9) closure_update<L, St, true, false, H>(a, n, live, v, w, xw);
-                else closure_update<L, St, false, false, H>(a, n, live, v, w, xw);
+                if (variant == 9) closure_update<L, St, true, false, H>(a, n, live, a.store != 0, v, w, xw);
+                else closure_update<L, St, false, false, H>(a, n, live, a.store != 0, v, w, xw);
             }
             if (live) scatter_node<L, St, false>(a, n, dd, v);
         }

@@ -22,12 +22,13 @@
 namespace lbmc {
 
 // H: the network with fp16 operands (else bf16)
+// store: the call stores rho / u
 template <class L, class St, bool GUO, bool RECORD, bool H>
-__device__ __forceinline__ void closure_update(const StepArgs<float> &a, int n, bool live, float (&v)[L::Q],
-                                               const MlpEval &w, uint4 *xw)
+__device__ __forceinline__ void closure_update(const StepArgs<float> &a, int n, bool live, bool store,
+                                               float (&v)[L::Q], const MlpEval &w, uint4 *xw)
 {
     constexpr int D = L::D;
-    const unsigned m = a.all_fluid ? 0u : ldg(a.mask + n);
+    const uint16_t desc = node_class(a, n);
     float F[3] = {0.f, 0.f, 0.f};
     if constexpr (GUO) {
         sfor<0, D>([&](auto dd) {
@@ -41,13 +42,13 @@ __device__ __forceinline__ void closure_update(const StepArgs<float> &a, int n, 
     fast_closure_features<L, St::shifted>(st, x);
     const float y = mlp_wave_eval<H>(w, xw, mlp_input_eval<H>(w.sc, x));
     if (!live) return;
-    if (m == 0) {
+    if (desc == 0) {
         float t = w.sc.out_a * y + w.sc.out_b + a.closure_shift;
         const bool in_band = t >= w.sc.lo && t <= w.sc.hi;
         if constexpr (RECORD) stg(a.tcache + n, in_band ? t : __builtin_nanf(""));
         if (!in_band) t = a.c_smag > 0.f ? fast_smag_tau<L, St::shifted>(st, a.tau, a.c_smag) : a.tau;
         fast_relax<L, St::shifted, GUO>(v, st, t, a.tau, F);
-        if (a.store) {
+        if (store) {
             sfor<0, D>([&](auto dd) {
                 constexpr int d = decltype(dd)::value;
                 stg(a.u[d] + n, st.u[d]);
@@ -55,7 +56,7 @@ __device__ __forceinline__ void closure_update(const StepArgs<float> &a, int n, 
             stg(a.rho + n, st.rho);
         }
     } else {
-        node_update<L, St, 0, GUO, true, false>(a, n, v);
+        node_update_as<L, St, 0, GUO, true, false>(a, n, desc, store, v);
     }
 }
 
@@ -63,9 +64,10 @@ __device__ __forceinline__ void closure_update(const StepArgs<float> &a, int n, 
 // recorded tau (the Smagorinsky tau of the current state where the record is
 // NaN); no network.
 template <class L, class St, bool GUO>
-__device__ __forceinline__ void closure_reuse_node(const StepArgs<float> &a, int n, float (&v)[L::Q])
+__device__ __forceinline__ void closure_reuse_node(const StepArgs<float> &a, int n, uint16_t desc, bool store,
+                                                   float (&v)[L::Q])
 {
-    if (a.all_fluid || ldg(a.mask + n) == 0) {
+    if (desc == 0) {
         constexpr int D = L::D;
         float F[3] = {0.f, 0.f, 0.f};
         if constexpr (GUO) {
@@ -79,7 +81,7 @@ __device__ __forceinline__ void closure_reuse_node(const StepArgs<float> &a, int
         float t = ldg(a.tcache + n);
         if (t != t) t = a.c_smag > 0.f ? fast_smag_tau<L, St::shifted>(st, a.tau, a.c_smag) : a.tau;
         fast_relax<L, St::shifted, GUO>(v, st, t, a.tau, F);
-        if (a.store) {
+        if (store) {
             sfor<0, D>([&](auto dd2) {
                 constexpr int d = decltype(dd2)::value;
                 stg(a.u[d] + n, st.u[d]);
@@ -87,7 +89,7 @@ __device__ __forceinline__ void closure_reuse_node(const StepArgs<float> &a, int
             stg(a.rho + n, st.rho);
         }
     } else {
-        node_update<L, St, 0, GUO, true, false>(a, n, v);
+        node_update_as<L, St, 0, GUO, true, false>(a, n, desc, store, v);
     }
 }
 
@@ -117,7 +119,7 @@ __global__ __launch_bounds__(kBlock, 4) void closure_step_kernel(const StepArgs<
         slot_offsets<L>(a, n, dd);
         float v[L::Q];
         gather_node<L, St, WIDE>(a, n, dd, v);
-        closure_update<L, St, GUO, RECORD, H>(a, n, live, v, w, xw);
+        closure_update<L, St, GUO, RECORD, H>(a, n, live, a.store != 0, v, w, xw);
         if (live) scatter_node<L, St, WIDE>(a, n, dd, v);
     }
 }
@@ -134,7 +136,7 @@ __global__ __launch_bounds__(kBlock) void closure_reuse_kernel(const StepArgs<fl
     slot_offsets<L>(a, n, dd);
     float v[L::Q];
     gather_node<L, St, WIDE>(a, n, dd, v);
-    closure_reuse_node<L, St, GUO>(a, n, v);
+    closure_reuse_node<L, St, GUO>(a, n, node_class(a, n), a.store != 0, v);
     scatter_node<L, St, WIDE>(a, n, dd, v);
 }
 

@@ -92,6 +92,9 @@ struct lbmc_ctx {
 
 namespace lbmc {
 
+// the state has moved to the second population buffer: it becomes the first
+void swap_populations(lbmc_ctx *c);
+
 // Kernel arguments of call t (the reference's iterate_kernel(..., t)).
 template <class C>
 inline void fill_args(const lbmc_ctx *c, StepArgs<C> &a, long long t, int store)

@@ -71,6 +71,16 @@ hipError_t launch_copy(const void *src, void *dst, size_t nbytes, hipStream_t s)
 hipError_t launch_batch_fp64(int lattice, const void *members, const int2 *chunks, int nchunks, int grid, int sub,
                              int lds, hipStream_t s);
 
+// passes of several calls over the D2Q9 members of a batch, and the closure
+// members' evaluating calls, batch_tile.hip, batch_tile_fp64.hip
+struct BatchPass;
+hipError_t launch_batch_tiles_fp64(const void *members, const int2 *tiles, int ntiles, const BatchPass &bp,
+                                   hipStream_t s);
+hipError_t launch_batch_tiles_fp32(const void *members, const int2 *tiles, int ntiles, const BatchPass &bp,
+                                   hipStream_t s);
+hipError_t launch_batch_call_fp32(const void *members, const int2 *chunks, int nchunks, int grid, int sub,
+                                  const void *mlp, bool record, bool fp16, const BatchPass &bp, hipStream_t s);
+
 // learned closure, mlp.hip: operand image of a model's current weights with
 // the fallback band, into device memory dst on stream s
 size_t mlp_image_bytes();

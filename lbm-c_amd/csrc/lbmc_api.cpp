@@ -474,6 +474,12 @@ hipError_t dev_malloc(void **p, size_t bytes)
     return freed ? hipMalloc(p, bytes) : e;
 }
 
+void swap_populations(lbmc_ctx *c)
+{
+    std::swap(c->f, c->f2);
+    drop_graph(c);  // captured with the other buffer
+}
+
 }  // namespace lbmc
 
 extern "C" {

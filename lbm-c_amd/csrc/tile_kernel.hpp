@@ -50,9 +50,11 @@ __device__ __forceinline__ int tile_slot(int id, int jx, int jy)
 }
 
 // One tile of a pass.  T threads, NPT nodes per thread, W * H <= T * NPT.
-template <class L, class St, int FAM, bool GUO, bool SMAG, int T, int NPT>
+// update(n, desc, store, v): the update of node n, class descriptor desc, on
+// its populations v.
+template <class L, class St, int T, int NPT, class Update>
 __device__ __forceinline__ void tile_calls(const StepArgs<typename St::C> &a, const TilePass &p, unsigned tile,
-                                           typename St::S *lds)
+                                           typename St::S *lds, Update &&update)
 {
     using C = typename St::C;
     using S = typename St::S;
@@ -144,7 +146,7 @@ __device__ __forceinline__ void tile_calls(const StepArgs<typename St::C> &a, co
             C v[G][Q];
             sfor<g0, g0 + G>([&](auto qq) {
                 constexpr int q = decltype(qq)::value;
-                if (depth(info[q]) >= 0) {
+                if (p.calls > 1 ? depth(info[q]) >= 0 : (info[q] & 0x100) != 0) {
                     int dx[3], dy[3];
                     const int n = index(node[q]);
                     offsets(n, p.rs, dx, dy);
@@ -162,8 +164,7 @@ __device__ __forceinline__ void tile_calls(const StepArgs<typename St::C> &a, co
                 const bool own = (info[q] & 0x100) != 0;
                 if (p.calls > 1 ? depth(info[q]) >= 0 : own) {
                     const int n = index(node[q]);
-                    node_update_as<L, St, FAM, GUO, SMAG, false>(a, n, (uint16_t)((unsigned)info[q] >> 16),
-                                                                 (p.store & 1u) != 0 && own, v[q - g0]);
+                    update(n, (uint16_t)((unsigned)info[q] >> 16), (p.store & 1u) != 0 && own, v[q - g0]);
                     if (p.calls > 1) to_lds((int)threadIdx.x + q * T, n, 0, 0, ts, v[q - g0]);
                     else to_dst(n, ts, v[q - g0]);
                 }
@@ -178,7 +179,7 @@ __device__ __forceinline__ void tile_calls(const StepArgs<typename St::C> &a, co
         });
         const int n = index(node[q]);
         const bool st = ((p.store >> j) & 1u) != 0 && (info[q] & 0x100) != 0;
-        node_update_as<L, St, FAM, GUO, SMAG, false>(a, n, (uint16_t)((unsigned)info[q] >> 16), st, v);
+        update(n, (uint16_t)((unsigned)info[q] >> 16), st, v);
         write(n, v);
     };
     // further calls: in LDS
@@ -209,7 +210,9 @@ template <class L, class St, int FAM, bool GUO, bool SMAG, int T, int NPT>
 __global__ __launch_bounds__(T, 4) void tile_kernel(const StepArgs<typename St::C> a, const TilePass p)
 {
     __shared__ typename St::S lds[L::Q * T * NPT];
-    tile_calls<L, St, FAM, GUO, SMAG, T, NPT>(a, p, blockIdx.x, lds);
+    tile_calls<L, St, T, NPT>(a, p, blockIdx.x, lds, [&](int n, uint16_t desc, bool st, typename St::C(&v)[L::Q]) {
+        node_update_as<L, St, FAM, GUO, SMAG, false>(a, n, desc, st, v);
+    });
 }
 
 }  // namespace lbmc

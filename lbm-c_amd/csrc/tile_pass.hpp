@@ -143,6 +143,17 @@ inline TilePlan plan_tiles(int Lx, int Ly, int slot_bytes, int ncu)
     return best;
 }
 
+// Work of a plan's tiles per call, in ns of one CU (tile_estimate's terms),
+// for batches, whose tiles of all members fill the chip together.
+inline double tile_work(const TilePlan &q, int slot_bytes)
+{
+    const double ns_node = slot_bytes == 8 ? 2.9 : slot_bytes == 4 ? 1.2 : 1.7;
+    double nodes = 0;
+    for (int j = 0; j <= q.M; j++) nodes += (double)(q.W - 2 * j) * (q.H - 2 * j);
+    const double bytes = 9 * (q.H * ((double)q.W * slot_bytes + 96) + q.OH * ((double)q.OW * slot_bytes + 96));
+    return (double)q.ntx * q.nty * (nodes * ns_node + 0.5 * bytes / 20) / (q.M + 1);
+}
+
 // the geometry half of a pass's arguments
 inline void tile_geometry(const TilePlan &q, const int *L, TilePass &p)
 {

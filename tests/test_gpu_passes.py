@@ -114,3 +114,51 @@ def test_march_planned_shape(monkeypatch, storage):
     got = _run(monkeypatch, case, storage, None, 5)
     for a, b in zip(got, want):
         assert np.array_equal(a, b)
+
+
+def _batch(monkeypatch, pass_env, storage, every, store_every, runs, swap_in=False):
+    """Uneven members (plain BGK, MRT with forcing, prescribed values and, when
+    every > 0, learned-closure members) stepped as a batch."""
+    if pass_env is None:
+        monkeypatch.delenv("LBMC_PASS", raising=False)
+    else:
+        monkeypatch.setenv("LBMC_PASS", pass_env)
+    group = [cases.channel_d2q9(37, 21, collision=cases.MRT, rates=cases.d2q9_rates(0.8)),
+             cases.channel_d2q9(130, 66), cases.pressure_d2q9(), cases.porous_d2q9(L=40, collision=cases.NTPOR),
+             cases.channel_d2q9(64, 48), cases.channel_d2q9(90, 31)]
+    lats = [cases.build(lbmc.Lattice, c, storage=storage) for c in group]
+    model = None
+    if every:
+        import pymlp
+        model = lbmc.Mlp(pymlp.flatten(pymlp.init_params(3)), mu=[0] * 6 + [1], isd=[300.0] * 6 + [100.0], out_a=0.02,
+                         out_b=0.8)
+        for lat in lats[4:]:
+            lat.set_closure(model, 0.6, 1.0)
+            lat.set_closure_interval(every)
+    b = lbmc.Batch(lats)
+    for t0, n in runs:
+        b.run(t0, n, store_every)
+        lats[1].step(t0 + n, False)  # a member on its own between batch runs
+        lats[1].step(t0 + n + 1, False)
+    out = []
+    for lat in lats:
+        rho, u = lat.get_macros()
+        out.append((lat.get_f(), rho, u))
+    b.close()
+    for lat in lats:
+        lat.close()
+    if model is not None:
+        model.close()
+    return out
+
+
+@pytest.mark.parametrize("storage,every", [(0, 0), (1, 0), (1, 1), (1, 2), (1, 4), (1, 8)],
+                         ids=["f64", "f32", "every1", "every2", "every4", "every8"])
+def test_batch_passes_match_one_call_per_launch(monkeypatch, storage, every):
+    runs = [(3, 41), (44, 1), (45, 18), (2 ** 31 + 7, 9)]
+    for store_every in (0, 4, 9):
+        want = _batch(monkeypatch, "0", storage, every, store_every, runs)
+        got = _batch(monkeypatch, None, storage, every, store_every, runs)
+        for k, (w, g) in enumerate(zip(want, got)):
+            for a, b in zip(g, w):
+                assert np.array_equal(a, b), (k, store_every)
