@@ -159,7 +159,7 @@ lbmc_status lbmc_set_f(lbmc_ctx *ctx, const double *const *f);
  * reference: it is for callers that cannot allocate device memory (code
  * between graph captures, tight serving or checkpoint loops, harnesses that
  * forbid hipMalloc).  lbmc_get_f allocates an N-double conversion buffer on
- * every call; this variant converts through a fixed 8 MiB device array
+ * every call unless the storage is FP64; this variant converts through a fixed 8 MiB device array
  * (1,048,576 doubles, one per GPU for the life of the process), one chunk of
  * at most that many slots of one direction at a time, so lattices of any
  * size are read with the same results, bit for bit.  Calls that overlap on

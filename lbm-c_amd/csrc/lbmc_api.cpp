@@ -16,6 +16,7 @@
 
 #include "../../include/lbmc.h"
 #include "dispatch.hpp"
+#include "host_copy.hpp"
 #include "lattice.hpp"
 #include "node_index.hpp"
 #include "step_args.hpp"
@@ -559,6 +560,7 @@ lbmc_status lbmc_create(const lbmc_desc *desc, lbmc_ctx **out)
         if (half) c->hs = N / 2;
     }
     choose_shape(c);
+    staging_hold();
     if (const char *env = getenv("LBMC_GRAPH")) c->use_graph = atoi(env) != 0;
 
     auto bail = [&](lbmc_status st) {
@@ -652,6 +654,7 @@ lbmc_status lbmc_destroy(lbmc_ctx *c)
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->stream) (void)hipStreamDestroy(c->stream);
+    staging_release();
     delete c;
     return LBMC_OK;
 }
@@ -902,23 +905,13 @@ lbmc_status lbmc_get_macros(lbmc_ctx *c, double *rho, double *const *u)
 {
     if (!c) return fail(nullptr, LBMC_ERR_INVALID, "null context");
     HIP_TRY(c, hipSetDevice(c->desc.device), "hipSetDevice");
-    HIP_TRY(c, hipStreamSynchronize(c->stream), "sync");
-    const size_t N = (size_t)c->N;
-    auto read = [&](const void *src, double *dst) -> lbmc_status {
-        if (!dst) return LBMC_OK;
-        if (c->cbytes == 8) {
-            HIP_TRY(c, hipMemcpy(dst, src, 8 * N, hipMemcpyDeviceToHost), "macro read");
-        } else {
-            std::vector<float> tmp(N);
-            HIP_TRY(c, hipMemcpy(tmp.data(), src, 4 * N, hipMemcpyDeviceToHost), "macro read");
-            for (size_t k = 0; k < N; k++) dst[k] = tmp[k];
-        }
-        return LBMC_OK;
-    };
-    if (lbmc_status st = read(c->rho, rho)) return st;
+    HostRead r[4];
+    int count = 0;
+    if (rho) r[count++] = HostRead{rho, c->rho, (size_t)c->N};
     if (u)
         for (int d = 0; d < c->D; d++)
-            if (lbmc_status st = read(c->u[d], u[d])) return st;
+            if (u[d]) r[count++] = HostRead{u[d], c->u[d], (size_t)c->N};
+    HIP_TRY(c, read_arrays(r, count, (int)c->cbytes, c->cbytes == 4, c->desc.device, c->stream), "macro read");
     return LBMC_OK;
 }
 
@@ -927,22 +920,13 @@ lbmc_status lbmc_get_node(lbmc_ctx *c, long long idx, double *rho, double *u)
     if (!c) return fail(nullptr, LBMC_ERR_INVALID, "null context");
     if (idx < 0 || idx >= c->N) return fail(c, LBMC_ERR_INVALID, "node %lld out of range", idx);
     HIP_TRY(c, hipSetDevice(c->desc.device), "hipSetDevice");
-    HIP_TRY(c, hipStreamSynchronize(c->stream), "sync");
-    auto read1 = [&](const void *base, double *dst) -> lbmc_status {
-        if (!dst) return LBMC_OK;
-        if (c->cbytes == 8) {
-            HIP_TRY(c, hipMemcpy(dst, (const double *)base + idx, 8, hipMemcpyDeviceToHost), "node read");
-        } else {
-            float v;
-            HIP_TRY(c, hipMemcpy(&v, (const float *)base + idx, 4, hipMemcpyDeviceToHost), "node read");
-            *dst = v;
-        }
-        return LBMC_OK;
-    };
-    if (lbmc_status st = read1(c->rho, rho)) return st;
+    HostRead r[4];
+    int count = 0;
+    const size_t at = (size_t)idx * c->cbytes;
+    if (rho) r[count++] = HostRead{rho, (const char *)c->rho + at, 1};
     if (u)
-        for (int d = 0; d < c->D; d++)
-            if (lbmc_status st = read1(c->u[d], &u[d])) return st;
+        for (int d = 0; d < c->D; d++) r[count++] = HostRead{&u[d], (const char *)c->u[d] + at, 1};
+    HIP_TRY(c, read_arrays(r, count, (int)c->cbytes, c->cbytes == 4, c->desc.device, c->stream), "node read");
     return LBMC_OK;
 }
 
@@ -950,14 +934,23 @@ lbmc_status lbmc_get_f(lbmc_ctx *c, double *const *f)
 {
     if (!c || !f) return fail(c, LBMC_ERR_INVALID, "null argument");
     HIP_TRY(c, hipSetDevice(c->desc.device), "hipSetDevice");
+    if (c->storage == LBMC_FP64) {
+        // the slots as they are
+        HostRead r[15];
+        int count = 0;
+        for (int i = 0; i < c->Q; i++)
+            if (f[i]) r[count++] = HostRead{f[i], (const double *)c->f + (size_t)i * (size_t)c->npad, (size_t)c->N};
+        HIP_TRY(c, read_arrays(r, count, 8, false, c->desc.device, c->stream), "get_f");
+        return LBMC_OK;
+    }
     double *tmp = nullptr;
     HIP_TRY(c, dev_malloc((void **)&tmp, sizeof(double) * (size_t)c->N), "f read buffer");
     hipError_t e = hipSuccess;
     for (int i = 0; i < c->Q && e == hipSuccess; i++) {
         if (!f[i]) continue;
         e = launch_f_to_double(c->desc.lattice, c->storage, c->f, c->npad, i, 0, c->N, c->hs, tmp, c->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-        if (e == hipSuccess) e = hipMemcpy(f[i], tmp, sizeof(double) * (size_t)c->N, hipMemcpyDeviceToHost);
+        const HostRead r{f[i], tmp, (size_t)c->N};
+        if (e == hipSuccess) e = read_arrays(&r, 1, 8, false, c->desc.device, c->stream);
     }
     (void)hipFree(tmp);
     if (e != hipSuccess) return hip_fail(c, e, "get_f");
@@ -1025,16 +1018,28 @@ lbmc_status lbmc_set_f(lbmc_ctx *c, const double *const *f)
     if (!c || !f) return fail(c, LBMC_ERR_INVALID, "null argument");
     invalidate_tau_record(c);
     HIP_TRY(c, hipSetDevice(c->desc.device), "hipSetDevice");
+    const size_t bytes = sizeof(double) * (size_t)c->N;
+    if (c->storage == LBMC_FP64) {
+        // the slots as they are
+        HostWrite w[15];
+        int count = 0;
+        for (int i = 0; i < c->Q; i++)
+            if (f[i]) w[count++] = HostWrite{(double *)c->f + (size_t)i * (size_t)c->npad, f[i], bytes};
+        HIP_TRY(c, write_arrays(w, count, c->desc.device, c->stream), "set_f");
+        return LBMC_OK;
+    }
     double *tmp = nullptr;
-    HIP_TRY(c, dev_malloc((void **)&tmp, sizeof(double) * (size_t)c->N), "f write buffer");
-    hipError_t e = hipStreamSynchronize(c->stream);
+    HIP_TRY(c, dev_malloc((void **)&tmp, bytes), "f write buffer");
+    hipError_t e = hipSuccess;
     for (int i = 0; i < c->Q && e == hipSuccess; i++) {
         if (!f[i]) continue;
-        e = hipMemcpy(tmp, f[i], sizeof(double) * (size_t)c->N, hipMemcpyHostToDevice);
+        const HostWrite w{tmp, f[i], bytes};
+        e = write_arrays(&w, 1, c->desc.device, c->stream);
         if (e == hipSuccess)
             e = launch_f_from_double(c->desc.lattice, c->storage, c->f, c->npad, i, c->N, c->hs, tmp, c->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     }
+    const hipError_t w = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess) e = w;
     (void)hipFree(tmp);
     if (e != hipSuccess) return hip_fail(c, e, "set_f");
     return LBMC_OK;

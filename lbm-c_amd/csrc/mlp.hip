@@ -16,6 +16,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <numeric>
 #include <random>
 #include <string>
@@ -23,6 +24,7 @@
 
 #include "../../include/lbmc.h"
 #include "dispatch.hpp"
+#include "host_copy.hpp"
 #include "mlp.hpp"
 
 namespace lbmc {
@@ -368,6 +370,11 @@ struct lbmc_mlp {
     long long S = 0;
     float *partial = nullptr;
     int pcap = 0;
+    // inputs and outputs of lbmc_mlp_forward, kept up to 64 MB; a call that
+    // finds another thread's in it, or is larger, allocates its own
+    std::mutex fwd_mu;
+    float *fwd = nullptr;
+    size_t fwd_cap = 0;
     double *lossacc = nullptr;
     long long adam_t = 0;
     bool eval_fp16 = false;  // evaluation with fp16 operands (default bf16)
@@ -508,6 +515,7 @@ lbmc_status lbmc_mlp_create(int device, const float *params, const lbmc_mlp_scal
         if (!std::isfinite(params[k])) return mfail(nullptr, LBMC_ERR_INVALID, "lbmc_mlp_create: parameter %d not finite", k);
     }
     lbmc_mlp *m = new lbmc_mlp();
+    staging_hold();
     m->device = device;
     fill_scalars(m->sc, sc);
     lbmc_status st = LBMC_OK;
@@ -543,10 +551,11 @@ void lbmc_mlp_destroy(lbmc_mlp *m)
     if (!m) return;
     (void)hipSetDevice(m->device);
     if (m->stream) (void)hipStreamSynchronize(m->stream);
-    void *bufs[] = {m->params, m->m1, m->m2, m->grad, m->img, m->feat, m->target, m->order, m->partial, m->lossacc};
+    void *bufs[] = {m->params, m->m1, m->m2, m->grad, m->img, m->feat, m->target, m->order, m->partial, m->lossacc, m->fwd};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     if (m->stream) (void)hipStreamDestroy(m->stream);
+    staging_release();
     delete m;
 }
 
@@ -590,10 +599,25 @@ lbmc_status lbmc_mlp_forward(lbmc_mlp *m, const float *feat, long long S, float 
     if (S == 0) return LBMC_OK;
     if (S > (1LL << 31) / 8) return mfail(m, LBMC_ERR_INVALID, "lbmc_mlp_forward: too many samples");
     MLP_HIP(m, hipSetDevice(m->device));
-    float *dx = nullptr, *dy = nullptr;
-    MLP_HIP(m, dev_malloc((void **)&dx, (size_t)S * 7 * sizeof(float)));
-    hipError_t e = dev_malloc((void **)&dy, (size_t)S * sizeof(float));
-    if (e == hipSuccess) e = hipMemcpyAsync(dx, feat, (size_t)S * 7 * sizeof(float), hipMemcpyHostToDevice, m->stream);
+    const size_t need = (size_t)S * 8 * sizeof(float);
+    std::unique_lock<std::mutex> lock(m->fwd_mu, std::try_to_lock);
+    const bool keep = lock.owns_lock() && need <= ((size_t)64 << 20);
+    float *buf = keep && m->fwd_cap >= need ? m->fwd : nullptr;
+    if (!buf) {
+        if (keep && m->fwd) {
+            (void)hipFree(m->fwd);
+            m->fwd = nullptr;
+            m->fwd_cap = 0;
+        }
+        MLP_HIP(m, dev_malloc((void **)&buf, need));
+        if (keep) {
+            m->fwd = buf;
+            m->fwd_cap = need;
+        }
+    }
+    float *const dx = buf, *const dy = buf + (size_t)S * 7;
+    const HostWrite in{dx, feat, (size_t)S * 7 * sizeof(float)};
+    hipError_t e = write_arrays(&in, 1, m->device, m->stream);
     if (e == hipSuccess) {
         if (m->eval_fp16)
             hipLaunchKernelGGL(mlp_forward_kernel<true>, dim3((unsigned)((S + 255) / 256)), dim3(256), 0, m->stream,
@@ -603,10 +627,10 @@ lbmc_status lbmc_mlp_forward(lbmc_mlp *m, const float *feat, long long S, float 
                                m->img, dx, S, dy);
         e = hipGetLastError();
     }
-    if (e == hipSuccess) e = hipMemcpyAsync(y, dy, (size_t)S * sizeof(float), hipMemcpyDeviceToHost, m->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
-    (void)hipFree(dx);
-    if (dy) (void)hipFree(dy);
+    const HostRead out{y, dy, (size_t)S};
+    if (e == hipSuccess) e = read_arrays(&out, 1, (int)sizeof(float), false, m->device, m->stream);
+    else (void)hipStreamSynchronize(m->stream);
+    if (!keep) (void)hipFree(buf);
     if (e != hipSuccess) return mfail(m, LBMC_ERR_DEVICE, "lbmc_mlp_forward: %s", hipGetErrorString(e));
     return LBMC_OK;
 }

@@ -287,9 +287,9 @@ class Lattice:
     # -- read-back
     def get_macros(self):
         rho = np.empty(self.n)
-        u = [np.empty(self.n) for _ in range(self.dim)]
-        self._check(_lib.lbmc_get_macros(self._h, _dptr(rho), _ptr_array(u, 3)))
-        return rho, np.stack(u)
+        u = np.empty((self.dim, self.n))
+        self._check(_lib.lbmc_get_macros(self._h, _dptr(rho), _ptr_array(list(u), 3)))
+        return rho, u
 
     def get_node(self, idx):
         rho = ct.c_double()
@@ -298,9 +298,9 @@ class Lattice:
         return rho.value, np.array(u[: self.dim])
 
     def get_f(self):
-        f = [np.empty(self.n) for _ in range(self.q)]
-        self._check(_lib.lbmc_get_f(self._h, _ptr_array(f, 15)))
-        return np.stack(f)
+        f = np.empty((self.q, self.n))
+        self._check(_lib.lbmc_get_f(self._h, _ptr_array(list(f), 15)))
+        return f
 
     def get_f_noalloc(self):
         """get_f through the library's fixed device scratch (no allocation)."""
