@@ -61,11 +61,11 @@ __device__ __forceinline__ void closure_update(const StepArgs<float> &a, int n, 
 }
 
 // A call between evaluations, one node: plain fluid nodes relax with the
-// recorded tau (the Smagorinsky tau of the current state where the record is
-// NaN); no network.
+// recorded tau t (the Smagorinsky tau of the current state where it is NaN);
+// no network.
 template <class L, class St, bool GUO>
-__device__ __forceinline__ void closure_reuse_node(const StepArgs<float> &a, int n, uint16_t desc, bool store,
-                                                   float (&v)[L::Q])
+__device__ __forceinline__ void closure_reuse_tau(const StepArgs<float> &a, int n, uint16_t desc, bool store, float t,
+                                                  float (&v)[L::Q])
 {
     if (desc == 0) {
         constexpr int D = L::D;
@@ -78,7 +78,6 @@ __device__ __forceinline__ void closure_reuse_node(const StepArgs<float> &a, int
         }
         FastState<L> st;
         fast_prepare<L, St::shifted, GUO>(v, F, st);
-        float t = ldg(a.tcache + n);
         if (t != t) t = a.c_smag > 0.f ? fast_smag_tau<L, St::shifted>(st, a.tau, a.c_smag) : a.tau;
         fast_relax<L, St::shifted, GUO>(v, st, t, a.tau, F);
         if (store) {
@@ -91,6 +90,14 @@ __device__ __forceinline__ void closure_reuse_node(const StepArgs<float> &a, int
     } else {
         node_update_as<L, St, 0, GUO, true, false>(a, n, desc, store, v);
     }
+}
+
+// the same with the record read here
+template <class L, class St, bool GUO>
+__device__ __forceinline__ void closure_reuse_node(const StepArgs<float> &a, int n, uint16_t desc, bool store,
+                                                   float (&v)[L::Q])
+{
+    closure_reuse_tau<L, St, GUO>(a, n, desc, store, desc == 0 ? ldg(a.tcache + n) : 0.f, v);
 }
 
 template <class L, class St, bool GUO, bool RECORD, bool WIDE, bool H>

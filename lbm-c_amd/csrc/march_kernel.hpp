@@ -28,10 +28,17 @@
 // twice; 32 x 28 has 12 % but is 11 % slower.  Three calls per pass (own 64
 // x 11, two barriers per plane) measured 251 us, two 512-thread blocks per CU
 // 257, non-temporal stores 244.
+//
+// The closure's calls between evaluations take the same passes: at 128^3 FP32
+// a call of an interval of 4 takes 41.9 us on average against 47.7 with one
+// call per launch, of 8 33.6 against 44.4 (200^3: 144 against 209).  The
+// evaluating calls stay alone: their network keeps the vector units busy (85 %
+// of their issue slots), and its registers beside the march's do not fit.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
+#include "closure_kernel.hpp"
 #include "step_kernel.hpp"
 #include "tile_pass.hpp"
 
@@ -48,8 +55,10 @@ __device__ __forceinline__ void arrived(C &x)
 constexpr int march_row(int i) { return i < 5 ? i - 1 : i - 3; }
 
 // T threads; CLS: the node classes of the lattice (MARCH_*).  One block per
-// CU: 4 waves per SIMD at 1024 threads, 2 at 512.
-template <class L, class St, int FAM, bool GUO, bool SMAG, bool MFIX, int CLS, int T>
+// CU: 4 waves per SIMD at 1024 threads, 2 at 512.  REUSE: calls of the
+// learned closure between evaluations (closure_reuse_tau); a column's record
+// of a plane is loaded once for both calls.
+template <class L, class St, int FAM, bool GUO, bool SMAG, bool MFIX, int CLS, int T, bool REUSE>
 __global__ __launch_bounds__(T, T / 256) void march_kernel(const StepArgs<typename St::C> a, const MarchPass p)
 {
     using C = typename St::C;
@@ -104,25 +113,36 @@ __global__ __launch_bounds__(T, T / 256) void march_kernel(const StepArgs<typena
             v[decltype(ii)::value] = St::load(ldg((const S *)slot(ii, p.src, p.rstride, p.rs, z, rx, ry)));
         });
     };
+    auto record = [&](int z) -> C { return ldg(a.tcache + (nxy + z * (int)plane)); };
     auto node_desc = [&](int n) -> uint16_t {
         if constexpr (CLS == MARCH_FLUID) return 0;
         else return ldg(a.mask + n) != 0 ? (uint16_t)CLS_SOLID : (uint16_t)0;
     };
 
+    // the update of node n; t: its recorded relaxation time
+    auto update = [&](int n, uint16_t desc, bool store, C t, C (&v)[Q]) {
+        if constexpr (REUSE) closure_reuse_tau<L, St, GUO>(a, n, desc, store, t, v);
+        else node_update_as<L, St, FAM, GUO, SMAG, MFIX>(a, n, desc, store, v);
+    };
+
     C flat[5], up1[5], up2[5];  // arrivals held for the second call: e_z = 0 of the last plane, e_z = +1 of the
                                 // last plane and of the one before it
     uint16_t d2 = 0;            // class descriptor of the last plane's node
+    C t1 = 0, t2 = 0;           // records of this plane's node and of the last plane's
     // plane k of the range: the first call there, on its populations f, and
     // the second call of plane k - 1; loads plane k + 1 into w meanwhile
     auto plane_calls = [&](int k, C (&f)[Q], C (&w)[Q]) {
         const int z = wrap_z(z0 + k);
         const int n = nxy + z * (int)plane;
         const uint16_t d1 = node_desc(n);
-        gather(wrap_z(z0 + min(k + 1, oz)), w);
+        const int zn = wrap_z(z0 + min(k + 1, oz));
+        gather(zn, w);
+        C tn = 0;
+        if constexpr (REUSE) tn = record(zn);
         __builtin_amdgcn_sched_barrier(0);
         S(*row)[T] = lds[k & 1];
         const bool st = (p.store & 1u) != 0 && own && k >= 0 && k < oz;
-        node_update_as<L, St, FAM, GUO, SMAG, MFIX>(a, n, d1, st, f);
+        update(n, d1, st, t1, f);
         sfor<1, Q>([&](auto ii) {
             constexpr int i = decltype(ii)::value;
             if constexpr (L::ex[i] != 0 || L::ey[i] != 0) row[march_row(i)][id] = St::store(f[i]);
@@ -147,7 +167,7 @@ __global__ __launch_bounds__(T, T / 256) void march_kernel(const StepArgs<typena
                 else if constexpr (L::ez[i] == 1) r[i] = up2[cu++];
                 else r[i] = arrive(ii);
             });
-            node_update_as<L, St, FAM, GUO, SMAG, MFIX>(a, ns, d2, (p.store & 2u) != 0, r);
+            update(ns, d2, (p.store & 2u) != 0, t2, r);
         }
         if (own) {
             int cf = 0, cu = 0;
@@ -172,12 +192,18 @@ __global__ __launch_bounds__(T, T / 256) void march_kernel(const StepArgs<typena
         // planes ahead fetch 1.45 GB per pass at 256^3 instead of 1.24 and
         // take 5 % longer.
         sfor<0, Q>([&](auto ii) { arrived(w[decltype(ii)::value]); });
+        if constexpr (REUSE) {
+            arrived(tn);
+            t2 = t1;
+            t1 = tn;
+        }
         d2 = d1;
     };
     // two sets of populations in turn, so that a load in flight stays in its
     // registers
     C va[Q], vb[Q];
     gather(wrap_z(z0 - 1), va);
+    if constexpr (REUSE) t1 = record(wrap_z(z0 - 1));
     sfor<0, Q>([&](auto ii) { arrived(va[decltype(ii)::value]); });
     for (int k = -1;; k += 2) {
         plane_calls(k, va, vb);

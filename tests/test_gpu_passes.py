@@ -162,3 +162,37 @@ def test_batch_passes_match_one_call_per_launch(monkeypatch, storage, every):
         for k, (w, g) in enumerate(zip(want, got)):
             for a, b in zip(g, w):
                 assert np.array_equal(a, b), (k, store_every)
+
+
+def _closure_run(monkeypatch, shape, case, every, store_every, band):
+    monkeypatch.setenv("LBMC_PASS", shape)
+    import pymlp
+    model = lbmc.Mlp(pymlp.flatten(pymlp.init_params(3)), mu=[0] * 6 + [1], isd=[300.0] * 6 + [100.0], out_a=0.02,
+                     out_b=0.8)
+    lat = cases.build(lbmc.Lattice, case, storage=1)
+    lat.set_closure(model, *band)
+    lat.set_closure_interval(every)
+    lat.run(3, 23, store_every)   # starts between evaluations, without a record
+    lat.run(26, 1, 1)
+    lat.run(27, every, 0)         # at most one pair: run one by one
+    lat.run(27 + every, 4 * every, 2)
+    f = lat.get_f()
+    lat.set_f(f)                  # the record goes with the state
+    lat.run(2 ** 31 + 2, 17, store_every)
+    rho, u = lat.get_macros()
+    out = lat.get_f(), rho, u
+    lat.close()
+    model.close()
+    return out
+
+
+@pytest.mark.parametrize("every", [2, 3, 4, 7, 8])
+@pytest.mark.parametrize("case", D3_CASES[:5], ids=lambda c: c["name"])
+def test_closure_passes_match_one_call_per_launch(monkeypatch, case, every):
+    # the band of the second leaves nodes outside: the record's NaN entries
+    for store_every, band in ((0, (0.6, 1.0)), (5, (0.799, 0.802))):
+        want = _closure_run(monkeypatch, "0", case, every, store_every, band)
+        for shape in ("37,13,3", "9,7,2", "64,8,1"):
+            got = _closure_run(monkeypatch, shape, case, every, store_every, band)
+            for a, b in zip(got, want):
+                assert np.array_equal(a, b), (shape, store_every)
