@@ -627,9 +627,17 @@ lbmc_status lbmc_mlp_forward(lbmc_mlp *m, const float *feat, long long S, float 
                                m->img, dx, S, dy);
         e = hipGetLastError();
     }
+    // outputs of 0.5-8 MB: into an array that has its pages hipMemcpy is ahead
+    // of the pieces (2 MB 132 us against 156), into a new one behind (451, 333)
+    const size_t bytes = (size_t)S * sizeof(float);
     const HostRead out{y, dy, (size_t)S};
-    if (e == hipSuccess) e = read_arrays(&out, 1, (int)sizeof(float), false, m->device, m->stream);
-    else (void)hipStreamSynchronize(m->stream);
+    if (e == hipSuccess) {
+        if (bytes > ((size_t)512 << 10) && bytes <= ((size_t)8 << 20))
+            e = hipMemcpyAsync(y, dy, bytes, hipMemcpyDeviceToHost, m->stream);
+        else e = read_arrays(&out, 1, (int)sizeof(float), false, m->device, m->stream);
+    }
+    const hipError_t idle = hipStreamSynchronize(m->stream);
+    if (e == hipSuccess) e = idle;
     if (!keep) (void)hipFree(buf);
     if (e != hipSuccess) return mfail(m, LBMC_ERR_DEVICE, "lbmc_mlp_forward: %s", hipGetErrorString(e));
     return LBMC_OK;
