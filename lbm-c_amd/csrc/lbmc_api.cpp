@@ -203,8 +203,8 @@ void drop_passes(lbmc_ctx *c)
 
 // Tiles of the passes over a lattice and their second population buffer:
 // lattices without sf nodes, D2Q9 ones whose direction arrays 32-bit offsets
-// reach, D3Q15 ones of fluid and solid nodes, BGK family, in 32 and 64 bits,
-// whose planes they reach.  The buffer is taken only while half of the device's memory stays
+// reach, D3Q15 ones of fluid and solid nodes in 32 and 64 bits whose planes
+// they reach.  The buffer is taken only while half of the device's memory stays
 // free, and given back when an allocation fails (dev_malloc), so that a
 // program's lattices fit as they would without it.
 void plan_passes(lbmc_ctx *c)
@@ -230,7 +230,7 @@ void plan_passes(lbmc_ctx *c)
             q.on = (long long)v[1] * v[2] <= cap.threads * cap.per_thread &&
                    tile_shape(c->L[0], c->L[1], v[0], v[1], v[2], v[3], q);
         }
-    } else if (c->D == 3 && c->key.family == 0 && slot >= 4 &&
+    } else if (c->D == 3 && slot >= 4 && march_takes(slot, c->key.family != 0, c->key.mfix != 0, c->key.guo != 0) &&
                (unsigned long long)c->L[0] * c->L[1] * slot < (1ULL << 31)) {
         c->march_cls = c->all_fluid ? MARCH_FLUID : MARCH_SOLID;
         bool plain = true;

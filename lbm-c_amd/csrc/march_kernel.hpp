@@ -58,11 +58,20 @@ constexpr int march_row(int i) { return i < 5 ? i - 1 : i - 3; }
 // CU: 4 waves per SIMD at 1024 threads, 2 at 512.  REUSE: calls of the
 // learned closure between evaluations (closure_reuse_tau); a column's record
 // of a plane is loaded once for both calls.
-template <class L, class St, int FAM, bool GUO, bool SMAG, bool MFIX, int CLS, int T, bool REUSE>
-__global__ __launch_bounds__(T, T / 256) void march_kernel(const StepArgs<typename St::C> a, const MarchPass p)
+// FORCE: MARCH_NO_FORCE, or a force per node or the same at every node.  The
+// last two are apart because a load of the force in an update waits, in the
+// one in-order counter, for the next plane's populations issued before it;
+// the compiler places that wait behind the branch that reads a uniform force
+// too.  With the load compiled out a forced BGK duct of 256^3 takes 244 us per
+// call in FP32 instead of 273, 535 in FP64 instead of 606.
+template <class L, class St, int FAM, int FORCE, bool SMAG, bool MFIX, int CLS, int T, bool REUSE>
+__global__ __launch_bounds__(T, T / 256) void march_kernel(const StepArgs<typename St::C> args, const MarchPass p)
 {
     using C = typename St::C;
     using S = typename St::S;
+    constexpr bool GUO = FORCE != MARCH_NO_FORCE;
+    StepArgs<C> a = args;
+    if constexpr (FORCE == MARCH_UNIFORM_FORCE) a.force[0] = a.force[1] = a.force[2] = nullptr;
     static_assert(L::D == 3 && !St::stochastic, "D3Q15, storage without conversions");
     constexpr int Q = L::Q;
     __shared__ S lds[2][12][T];  // of even and odd planes: one barrier per plane
@@ -114,35 +123,37 @@ __global__ __launch_bounds__(T, T / 256) void march_kernel(const StepArgs<typena
         });
     };
     auto record = [&](int z) -> C { return ldg(a.tcache + (nxy + z * (int)plane)); };
-    auto node_desc = [&](int n) -> uint16_t {
+    auto solid = [&](int z) -> unsigned {
         if constexpr (CLS == MARCH_FLUID) return 0;
-        else return ldg(a.mask + n) != 0 ? (uint16_t)CLS_SOLID : (uint16_t)0;
+        else return ldg(a.mask + (nxy + z * (int)plane));
     };
 
-    // the update of node n; t: its recorded relaxation time
-    auto update = [&](int n, uint16_t desc, bool store, C t, C (&v)[Q]) {
-        if constexpr (REUSE) closure_reuse_tau<L, St, GUO>(a, n, desc, store, t, v);
-        else node_update_as<L, St, FAM, GUO, SMAG, MFIX>(a, n, desc, store, v);
+    // the update of node n; m, t: its mask byte and recorded relaxation time
+    // (the two classes apart, each compiled for its descriptor)
+    auto update = [&](int n, unsigned m, bool store, C t, C (&v)[Q]) {
+        if (CLS != MARCH_FLUID && m != 0) node_update_as<L, St, FAM, GUO, SMAG, MFIX>(a, n, (uint16_t)CLS_SOLID, store, v);
+        else if constexpr (REUSE) closure_reuse_tau<L, St, GUO>(a, n, 0, store, t, v);
+        else node_update_as<L, St, FAM, GUO, SMAG, MFIX>(a, n, 0, store, v);
     };
 
     C flat[5], up1[5], up2[5];  // arrivals held for the second call: e_z = 0 of the last plane, e_z = +1 of the
                                 // last plane and of the one before it
-    uint16_t d2 = 0;            // class descriptor of the last plane's node
-    C t1 = 0, t2 = 0;           // records of this plane's node and of the last plane's
+    unsigned m1 = 0, m2 = 0;    // mask bytes of this plane's node and of the last plane's, and
+    C t1 = 0, t2 = 0;           // their records: loaded a plane ahead like the populations
     // plane k of the range: the first call there, on its populations f, and
     // the second call of plane k - 1; loads plane k + 1 into w meanwhile
     auto plane_calls = [&](int k, C (&f)[Q], C (&w)[Q]) {
         const int z = wrap_z(z0 + k);
         const int n = nxy + z * (int)plane;
-        const uint16_t d1 = node_desc(n);
         const int zn = wrap_z(z0 + min(k + 1, oz));
         gather(zn, w);
+        unsigned mn = solid(zn);
         C tn = 0;
         if constexpr (REUSE) tn = record(zn);
         __builtin_amdgcn_sched_barrier(0);
         S(*row)[T] = lds[k & 1];
         const bool st = (p.store & 1u) != 0 && own && k >= 0 && k < oz;
-        update(n, d1, st, t1, f);
+        update(n, m1, st, t1, f);
         sfor<1, Q>([&](auto ii) {
             constexpr int i = decltype(ii)::value;
             if constexpr (L::ex[i] != 0 || L::ey[i] != 0) row[march_row(i)][id] = St::store(f[i]);
@@ -167,7 +178,7 @@ __global__ __launch_bounds__(T, T / 256) void march_kernel(const StepArgs<typena
                 else if constexpr (L::ez[i] == 1) r[i] = up2[cu++];
                 else r[i] = arrive(ii);
             });
-            update(ns, d2, (p.store & 2u) != 0, t2, r);
+            update(ns, m2, (p.store & 2u) != 0, t2, r);
         }
         if (own) {
             int cf = 0, cu = 0;
@@ -197,12 +208,15 @@ __global__ __launch_bounds__(T, T / 256) void march_kernel(const StepArgs<typena
             t2 = t1;
             t1 = tn;
         }
-        d2 = d1;
+        if constexpr (CLS != MARCH_FLUID) arrived(mn);
+        m2 = m1;
+        m1 = mn;
     };
     // two sets of populations in turn, so that a load in flight stays in its
     // registers
     C va[Q], vb[Q];
     gather(wrap_z(z0 - 1), va);
+    m1 = solid(wrap_z(z0 - 1));
     if constexpr (REUSE) t1 = record(wrap_z(z0 - 1));
     sfor<0, Q>([&](auto ii) { arrived(va[decltype(ii)::value]); });
     for (int k = -1;; k += 2) {

@@ -33,6 +33,9 @@ struct TilePass {
 // and measured 0.5-1.0 of one call per launch.
 enum { MARCH_FLUID = 0, MARCH_SOLID = 1 };
 
+// How a march kernel has its body force (march_kernel.hpp)
+enum { MARCH_NO_FORCE = 0, MARCH_NODE_FORCE = 1, MARCH_UNIFORM_FORCE = 2 };
+
 // Two calls of a D3Q15 lattice
 struct MarchPass {
     const void *src;
@@ -177,6 +180,16 @@ inline void tile_geometry(const TilePlan &q, const int *L, TilePass &p)
 // in 64 bits).
 constexpr int march_threads(int slot_bytes) { return slot_bytes == 8 ? 512 : 1024; }
 
+// Collisions that the march kernels take: all but the MRT family with its
+// inverse matrix (mfix) and a body force in 32 bits.  That update needs more
+// than the 128 registers of a 1024-thread block (measured 131 x 97 x 75 25.0 us
+// per call alone against 27.1 in passes, 256^3 363 against 391; without the
+// force 24.4 against 17.1 and 359 against 254).
+constexpr bool march_takes(int slot_bytes, bool mrt, bool mfix, bool force)
+{
+    return !(slot_bytes == 4 && mrt && mfix && force);
+}
+
 inline void march_shape(const int *L, int W, int H, int nz, TilePlan &q)
 {
     q.M = 1;
@@ -224,11 +237,13 @@ inline double march_step_estimate(double nodes, int slot_bytes)
 // 256 CUs).
 // Measured, us per call, one call per launch -> passes: FP32 BGK with
 // Smagorinsky, all fluid, 256^3 357 -> 230, 512^3 3005 -> 1774, 128^3 39.1 ->
-// 26, 131 x 97 x 75 21.6 -> 13.5; forced duct with solid walls 256^3 373 ->
-// 273, 131 x 97 x 75 23.9 -> 17.6; FP64 256^3 771 -> 551, 200 x 150 x 100
-// 137 -> 109; 64^3 6.2 against 8.3 in passes (not planned).  FP64 lattices
-// that fit the last-level cache once but not twice stay with one call per
-// launch (128^3: 74.6 against 75.0).  16-bit lattices have no passes: 256^3
+// 26, 131 x 97 x 75 21.6 -> 13.5; forced duct with solid walls 256^3 366 ->
+// 241, 131 x 97 x 75 24.0 -> 15.2; FP64 256^3 771 -> 551, 200 x 150 x 100
+// 137 -> 109; MRT, forced duct, FP64 131 x 97 x 75 42 -> 37, 200^3 402 -> 280;
+// MRT box FP32 256^3 359 -> 254; 64^3 6.2 against 8.3 in passes (not planned).
+// FP64 lattices that fit the last-level cache once but not twice stay with one
+// call per launch (128^3: BGK box 73.6 against 74.8, forced ducts 75 against
+// 80-97; only boxes of 150-220 MB would gain, 5-15 %).  16-bit lattices have no passes: 256^3
 // 192 us against 221, bound by the arithmetic that a pass repeats at the sides.
 inline TilePlan plan_march(const int *L, int slot_bytes, int ncu)
 {

@@ -82,7 +82,7 @@ D3_CASES = [
     cases.turbulence_d3q15(13, forcing=True),
     _duct(False),
     _duct(True),
-    cases.turbulence_d3q15(12, collision=cases.MRT),  # no passes: the hook changes nothing
+    cases.turbulence_d3q15(12, collision=cases.MRT),
     cases.faces_d3q15(),                              # boundary nodes: no passes either
 ]
 
@@ -98,6 +98,28 @@ def test_march_matches_one_call_per_launch(monkeypatch, case, storage):
             got = _run(monkeypatch, case, storage, shape, store_every)
             for a, b in zip(got, want):
                 assert np.array_equal(a, b), (shape, store_every)
+
+
+def _forced(case, uniform, collision, quirks):
+    n = len(case["fields"]["geometry"])
+    force = [np.full(n, 2e-5), np.full(n, -1e-6), np.zeros(n)] if uniform else case["fields"]["force"]
+    rates = cases.d3q15_rates(0.7) if collision == cases.MRT else None
+    return dict(case, desc=dict(case["desc"], collision_type=collision, quirks=quirks, tau_mrt=rates),
+                fields=dict(case["fields"], force=force))
+
+
+@pytest.mark.parametrize("storage", [0, 1], ids=["f64", "f32"])
+@pytest.mark.parametrize("quirks", [0, 3])
+@pytest.mark.parametrize("force", ["none", "node", "uniform"])
+@pytest.mark.parametrize("collision", [cases.BGK, cases.MRT], ids=["bgk", "mrt"])
+def test_march_of_forced_ducts(monkeypatch, collision, force, quirks, storage):
+    # every kernel of the march: collision, force, MRT matrix; walls inside
+    case = _forced(_duct(force != "none"), force == "uniform", collision, quirks)
+    want = _run(monkeypatch, case, storage, "0", 4)
+    for shape in ("37,13,3", "9,7,2"):
+        got = _run(monkeypatch, case, storage, shape, 4)
+        for a, b in zip(got, want):
+            assert np.array_equal(a, b), shape
 
 
 @pytest.mark.parametrize("storage", [0, 1], ids=["f64", "f32"])
