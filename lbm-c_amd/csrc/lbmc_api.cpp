@@ -220,11 +220,13 @@ void plan_passes(lbmc_ctx *c)
     const char *env = getenv("LBMC_PASS");
     int v[4] = {0, 0, 0, 0};
     const int nv = env ? sscanf(env, "%d,%d,%d,%d", &v[0], &v[1], &v[2], &v[3]) : 0;
+    bool plain = true;  // fluid and solid nodes only
+    for (int k = 1; k < c->ncls; k++) plain = plain && c->cls_host[k] == CLS_SOLID;
     if (c->nsf) {
         // the sf gather reads the state before every call
     } else if (c->D == 2 && !c->offsets64) {
         if (!env) {
-            q = plan_tiles(c->L[0], c->L[1], slot, ncu);
+            q = plan_tiles(c->L[0], c->L[1], slot, ncu, plain);
         } else if (nv == 4 && v[0] >= 0 && v[0] <= 2 && v[3] < 32) {
             const TileCapacity cap = tile_capacity(v[0], slot);
             q.on = (long long)v[1] * v[2] <= cap.threads * cap.per_thread &&
@@ -233,8 +235,6 @@ void plan_passes(lbmc_ctx *c)
     } else if (c->D == 3 && slot >= 4 && march_takes(slot, c->key.family != 0, c->key.mfix != 0, c->key.guo != 0) &&
                (unsigned long long)c->L[0] * c->L[1] * slot < (1ULL << 31)) {
         c->march_cls = c->all_fluid ? MARCH_FLUID : MARCH_SOLID;
-        bool plain = true;
-        for (int k = 1; k < c->ncls; k++) plain = plain && c->cls_host[k] == CLS_SOLID;
         if (!plain) {
             // boundary or porous nodes: one call per launch
         } else if (!env) {

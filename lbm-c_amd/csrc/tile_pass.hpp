@@ -125,12 +125,16 @@ inline double tile_estimate(const TilePlan &q, int slot_bytes, int ncu)
 // 161 -> 78).  The 16-bit one-call kernels move half of FP32's bytes and are
 // bound by the same arithmetic plus the conversions, so passes win only
 // where launches count: 64 x 48 3.4 -> 1.2, 1500 x 400 11.6 -> 8.0, 2786 x
-// 681 equal, 3392 x 3392 80 -> 92; hence the line at 2^20 nodes.
+// 681 equal, 3392 x 3392 80 -> 92; hence the line at 2^20 nodes.  Nodes of
+// other classes than fluid and solid (boundary, prescribed or porous: plain
+// false) cost more where tiles recompute them: MRT between pressure faces 640
+// x 500 8.75 -> 6.7, 800 x 640 11.9 against 14.6, 1000 x 1000 16.5 against
+// 17.2; hence 400 000 nodes there.
 // M up to 7: deeper passes of the small tiles recompute more than they save.
-inline TilePlan plan_tiles(int Lx, int Ly, int slot_bytes, int ncu)
+inline TilePlan plan_tiles(int Lx, int Ly, int slot_bytes, int ncu, bool plain)
 {
     TilePlan best;
-    if (slot_bytes == 2 && (long long)Lx * Ly > (1LL << 20)) return best;
+    if (slot_bytes == 2 && (long long)Lx * Ly > (plain ? 1LL << 20 : 400000LL)) return best;
     for (int size = 0; size <= 2; size++) {
         const TileCapacity cap = tile_capacity(size, slot_bytes);
         const int P = cap.threads * cap.per_thread;
