@@ -605,7 +605,6 @@ lbmc_status lbmc_create(const lbmc_desc *desc, lbmc_ctx **out)
         if (half) c->hs = N / 2;
     }
     choose_shape(c);
-    staging_hold();
     if (const char *env = getenv("LBMC_GRAPH")) c->use_graph = atoi(env) != 0;
 
     auto bail = [&](lbmc_status st) {
@@ -614,6 +613,7 @@ lbmc_status lbmc_create(const lbmc_desc *desc, lbmc_ctx **out)
         return st;
     };
     hipError_t e = hipSetDevice(desc->device);
+    staging_hold();  // on this device: a process that uses one touches no other
     if (e != hipSuccess) return bail(hip_fail(c, e, "hipSetDevice"));
     if ((e = hipStreamCreate(&c->stream)) != hipSuccess)
         return bail(hip_fail(c, e, "hipStreamCreate"));

@@ -515,7 +515,6 @@ lbmc_status lbmc_mlp_create(int device, const float *params, const lbmc_mlp_scal
         if (!std::isfinite(params[k])) return mfail(nullptr, LBMC_ERR_INVALID, "lbmc_mlp_create: parameter %d not finite", k);
     }
     lbmc_mlp *m = new lbmc_mlp();
-    staging_hold();
     m->device = device;
     fill_scalars(m->sc, sc);
     lbmc_status st = LBMC_OK;
@@ -523,6 +522,7 @@ lbmc_status lbmc_mlp_create(int device, const float *params, const lbmc_mlp_scal
         if (e != hipSuccess && st == LBMC_OK) st = mfail(nullptr, LBMC_ERR_DEVICE, "%s: %s", what, hipGetErrorString(e));
     };
     chk(hipSetDevice(device), "hipSetDevice");
+    staging_hold();
     chk(hipStreamCreate(&m->stream), "hipStreamCreate");
     chk(dev_malloc((void **)&m->params, MLP_NPARAM * sizeof(float)), "hipMalloc");
     chk(dev_malloc((void **)&m->m1, MLP_NPARAM * sizeof(float)), "hipMalloc");
