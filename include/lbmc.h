@@ -267,8 +267,9 @@ lbmc_status lbmc_set_closure_shift(lbmc_ctx *ctx, double dtau);
 /* ---- Batches of lattices ---------------------------------------------------
  *
  * Steps an ensemble of independent lattices of different sizes together:
- * one persistent launch per time step covers every member's nodes, and runs
- * are replayed from a captured HIP graph.  The reference steps one lattice
+ * D2Q9 members in 32 or 64 bits take several calls per launch (as lbmc_run
+ * does); otherwise one persistent launch per time step covers every member's
+ * nodes, and runs are replayed from a captured HIP graph.  The reference steps one lattice
  * per process (LBM-C/index.cu:102-108 calling iterate, :284-313); a batch is
  * an addition.  Members are contexts made by lbmc_create and set up as usual
  * (fields and initial state); they share lattice type, storage and device,
