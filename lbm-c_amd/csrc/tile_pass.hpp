@@ -125,17 +125,22 @@ inline double tile_estimate(const TilePlan &q, int slot_bytes, int ncu)
 // 161 -> 78).  The 16-bit one-call kernels move half of FP32's bytes and are
 // bound by the same arithmetic plus the conversions, so passes win only
 // where launches count: 64 x 48 3.4 -> 1.2, 1500 x 400 11.6 -> 8.0, 2786 x
-// 681 equal, 3392 x 3392 80 -> 92; hence the line at 2^20 nodes.  Nodes of
-// other classes than fluid and solid (boundary, prescribed or porous: plain
-// false) cost more where tiles recompute them: MRT between pressure faces 640
-// x 500 8.75 -> 6.7, 800 x 640 11.9 against 14.6, 1000 x 1000 16.5 against
-// 17.2; hence 400 000 nodes there.
+// 681 equal, 3392 x 3392 80 -> 92; hence the line at 2^20 nodes.
+// Lattices with nodes of other classes than fluid and solid (boundary,
+// prescribed or porous: plain false) take tiles of up to 512 nodes below 1.5e6
+// nodes in 16 and 32 bits: a tile that holds such nodes takes longer, and of a
+// few rounds of large tiles the last waits for it (MRT between pressure faces,
+// tiles of 2048 -> 512 nodes: FP32 512 x 512 7.4 -> 5.4, 1148 x 450 9.3 -> 7.5,
+// 1222 x 1000 15.4 -> 13.4, 1400 x 1400 19.6 against 19.0-19.9; FP16S 800 x 640
+// 14.6 -> 8.4, one call per launch 11.9; 64 bits hold 1024 and gain 0-5 %).
 // M up to 7: deeper passes of the small tiles recompute more than they save.
 inline TilePlan plan_tiles(int Lx, int Ly, int slot_bytes, int ncu, bool plain)
 {
     TilePlan best;
-    if (slot_bytes == 2 && (long long)Lx * Ly > (plain ? 1LL << 20 : 400000LL)) return best;
-    for (int size = 0; size <= 2; size++) {
+    const long long nodes = (long long)Lx * Ly;
+    if (slot_bytes == 2 && nodes > (1LL << 20)) return best;
+    const int largest = !plain && slot_bytes <= 4 && nodes < 1500000 ? 1 : 2;
+    for (int size = 0; size <= largest; size++) {
         const TileCapacity cap = tile_capacity(size, slot_bytes);
         const int P = cap.threads * cap.per_thread;
         for (int W = 16; W <= 128; W *= 2)

@@ -51,6 +51,16 @@ def test_passes_match_one_call_per_launch(monkeypatch, case, storage):
                 assert np.array_equal(a, b), (shape, store_every)
 
 
+@pytest.mark.parametrize("storage", [1, 2], ids=["f32", "f16s"])
+def test_planned_shape_between_pressure_faces(monkeypatch, storage):
+    # large enough that the planner limits the tiles of a lattice with boundary nodes
+    case = cases.pressure_d2q9(Lx=701, Ly=397, collision=cases.MRT)
+    want = _run(monkeypatch, case, storage, "0", 5)
+    got = _run(monkeypatch, case, storage, None, 5)
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)
+
+
 def test_long_time_index_and_late_start(monkeypatch):
     case = cases.channel_d2q9(37, 21)
     want = _run(monkeypatch, case, 0, "0", 3, t0=2 ** 31 + 5)
