@@ -185,7 +185,7 @@ inline void tile_geometry(const TilePlan &q, const int *L, TilePass &p)
 }
 
 // Threads per block of the march kernels, by the registers that a column
-// needs: 128 are available at 1024 threads (102-125 used), 256 at 512 (202-245
+// needs: 128 are available at 1024 threads (101-128 used), 256 at 512 (161-250
 // in 64 bits).
 constexpr int march_threads(int slot_bytes) { return slot_bytes == 8 ? 512 : 1024; }
 
