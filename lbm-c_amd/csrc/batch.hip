@@ -61,6 +61,7 @@ struct lbmc_batch {
     int nchunks = 0;
     int2 *cchunks = nullptr;  // the closure members' chunks
     int ncchunks = 0;
+    std::vector<char> chunk_closure;  // which members cchunks holds
     int eval_grid = 0;        // blocks of the evaluation kernel
     int *any_eval = nullptr;  // device flags [kBatchWindow]: some closure member evaluates call t_next + j
     const void *mlp = nullptr;  // closure weights shared by the closure members (a member's image)
@@ -270,39 +271,79 @@ static void xcd_order(std::vector<int2> &v, unsigned glog)
     v.swap(out);
 }
 
-// Chunk lists for `sub` tiles per chunk: (member, first node) of every
-// chunk, member by member, and the same for the closure members alone, in
-// XCD order with runs of ~1024 nodes (measured best for single D2Q9
-// lattices: 4 chunks of 256 nodes per XCD).
-lbmc_status build_chunks(lbmc_batch *b, int sub)
+// Chunk list for `sub` tiles per chunk: (member, first node) of every chunk,
+// member by member (the closure members alone: closure), in XCD order with
+// runs of ~1024 nodes (measured best for single D2Q9 lattices: 4 chunks of
+// 256 nodes per XCD).  Null without chunks.
+lbmc_status upload_chunks(lbmc_batch *b, int sub, bool closure, int2 **list, int *count)
 {
     const long long cn = (long long)sub * kBlock;
-    std::vector<int2> ch, cc;
-    for (int k = 0; k < b->count; k++)
-        for (long long n = 0; n < b->members[(size_t)k]->N; n += cn) {
-            ch.push_back(make_int2(k, (int)n));
-            if (b->members[(size_t)k]->key.closure) cc.push_back(make_int2(k, (int)n));
-        }
-    const unsigned glog = sub == 1 ? 2u : sub == 2 ? 1u : 0u;
-    xcd_order(ch, glog);
-    xcd_order(cc, glog);
-    if (b->chunks) B_HIP(b, hipFree(b->chunks));
-    if (b->cchunks) B_HIP(b, hipFree(b->cchunks));
-    b->chunks = nullptr;
-    b->cchunks = nullptr;
-    B_HIP(b, dev_malloc((void **)&b->chunks, sizeof(int2) * ch.size()));
-    B_HIP(b, hipMemcpy(b->chunks, ch.data(), sizeof(int2) * ch.size(), hipMemcpyHostToDevice));
-    if (!cc.empty()) {
-        B_HIP(b, dev_malloc((void **)&b->cchunks, sizeof(int2) * cc.size()));
-        B_HIP(b, hipMemcpy(b->cchunks, cc.data(), sizeof(int2) * cc.size(), hipMemcpyHostToDevice));
+    std::vector<int2> ch;
+    for (int k = 0; k < b->count; k++) {
+        const lbmc_ctx *c = b->members[(size_t)k];
+        if (closure && !c->key.closure) continue;
+        for (long long n = 0; n < c->N; n += cn) ch.push_back(make_int2(k, (int)n));
     }
-    b->nchunks = (int)ch.size();
-    b->ncchunks = (int)cc.size();
+    xcd_order(ch, sub == 1 ? 2u : sub == 2 ? 1u : 0u);
+    *list = nullptr;
+    *count = (int)ch.size();
+    if (ch.empty()) return LBMC_OK;
+    B_HIP(b, dev_malloc((void **)list, sizeof(int2) * ch.size()));
+    const hipError_t e = hipMemcpy(*list, ch.data(), sizeof(int2) * ch.size(), hipMemcpyHostToDevice);
+    if (e == hipSuccess) return LBMC_OK;
+    (void)hipFree(*list);
+    return bfail(b, LBMC_ERR_DEVICE, "chunk list: %s", hipGetErrorString(e));
+}
+
+// the closure members' chunks; the old list stays when there is no memory
+lbmc_status build_closure_chunks(lbmc_batch *b, int sub)
+{
+    int2 *list;
+    int count;
+    if (lbmc_status st = upload_chunks(b, sub, true, &list, &count)) return st;
+    if (b->cchunks) (void)hipFree(b->cchunks);
+    b->cchunks = list;
+    b->ncchunks = count;
+    b->chunk_closure.clear();
+    for (const lbmc_ctx *c : b->members) b->chunk_closure.push_back(c->key.closure ? 1 : 0);
+    // evaluation kernel: persistent, 4 blocks per CU (its residency)
+    b->eval_grid = std::max(1, std::min(count, 4 * b->ncu));
+    return LBMC_OK;
+}
+
+lbmc_status build_chunks(lbmc_batch *b, int sub)
+{
+    int2 *list;
+    int count;
+    if (lbmc_status st = upload_chunks(b, sub, false, &list, &count)) return st;
+    if (lbmc_status st = build_closure_chunks(b, sub)) {
+        (void)hipFree(list);
+        return st;
+    }
+    if (b->chunks) (void)hipFree(b->chunks);
+    b->chunks = list;
+    b->nchunks = count;
     b->sub = sub;
     b->grid = std::min(b->grid, b->nchunks);
-    // evaluation kernel: persistent, 4 blocks per CU (its residency)
-    b->eval_grid = std::max(1, std::min(b->ncchunks, 4 * b->ncu));
     return LBMC_OK;
+}
+
+// The closure members as they are now: a member's closure may be switched
+// between runs.  Their chunks, and the weights of one of them; the captured
+// graph holds both.
+lbmc_status follow_closures(lbmc_batch *b)
+{
+    std::vector<char> closure;
+    const void *mlp = b->mlp;
+    for (const lbmc_ctx *c : b->members) {
+        closure.push_back(c->key.closure ? 1 : 0);
+        if (c->key.closure && c->closure_model == b->closure_model) mlp = c->mlp_img;
+    }
+    if (mlp != b->mlp) drop_batch_graph(b);
+    b->mlp = mlp;
+    if (closure == b->chunk_closure) return LBMC_OK;
+    drop_batch_graph(b);
+    return build_closure_chunks(b, b->sub);
 }
 
 // ---- passes of several calls (D2Q9 members in 32 or 64 bits that all hold a
@@ -623,6 +664,7 @@ lbmc_status lbmc_batch_run(lbmc_batch *b, long long t0, int nsteps, int store_ev
     if (!b || nsteps < 0 || t0 < 0) return bfail(b, LBMC_ERR_INVALID, "lbmc_batch_run: bad argument");
     B_HIP(b, hipSetDevice(b->device));
     lbmc_status st = sync_members(b);
+    if (st == LBMC_OK) st = follow_closures(b);
     bool done = false;
     if (st == LBMC_OK) st = run_in_passes(b, t0, nsteps, store_every, false, &done);
     if (st == LBMC_OK && !done) st = upload(b, t0, store_every);
@@ -638,6 +680,7 @@ lbmc_status lbmc_batch_time_steps(lbmc_batch *b, long long t0, int nsteps, int s
     if (!b || nsteps <= 0 || t0 < 0 || !ms) return bfail(b, LBMC_ERR_INVALID, "lbmc_batch_time_steps: bad argument");
     B_HIP(b, hipSetDevice(b->device));
     lbmc_status st = sync_members(b);
+    if (st == LBMC_OK) st = follow_closures(b);
     bool done = false;
     if (st == LBMC_OK) st = run_in_passes(b, t0, nsteps, store_every, true, &done);
     if (st == LBMC_OK && !done) st = upload(b, t0, store_every);  // outside the timed region

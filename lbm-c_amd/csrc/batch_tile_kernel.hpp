@@ -125,6 +125,7 @@ __global__ __launch_bounds__(kBlock, 4) void batch_call_kernel(const BatchTileMe
         const int2 ch = chunks[c];
         if (ch.x < 0) continue;
         const BatchTileMember<float> &m = members[ch.x];
+        if (m.variant < 8) continue;  // not a closure member; block-uniform
         const StepArgs<float> &a = m.a;
         S *const f = (S *)(bp.odd ? m.p.dst : (void *)m.p.src);
         const int sx = call_shift(a, 0, bp.offset), sy = call_shift(a, 1, bp.offset);
