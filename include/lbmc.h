@@ -140,6 +140,12 @@ lbmc_status lbmc_step(lbmc_ctx *ctx, long long t, int store_macros);
  * of the library does not fit; the results do not depend on it. */
 lbmc_status lbmc_run(lbmc_ctx *ctx, long long t0, int nsteps, int store_every);
 
+/* How lbmc_run takes a lattice's calls: *calls per pass over memory, in tiles
+ * of *width x *height nodes or columns, margins included (1, 0 and 0: one
+ * call per launch).  Changes with lbmc_set_fields, and to one call per launch
+ * when the second population array is given back.  Any pointer may be NULL. */
+lbmc_status lbmc_pass_info(lbmc_ctx *ctx, int *calls, int *width, int *height);
+
 /* As lbmc_run, timed with HIP events on the context's stream; *ms is the
  * device time of the nsteps calls. */
 lbmc_status lbmc_time_steps(lbmc_ctx *ctx, long long t0, int nsteps, int store_every, float *ms);

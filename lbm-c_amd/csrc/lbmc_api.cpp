@@ -1176,6 +1176,17 @@ lbmc_status lbmc_info(const lbmc_ctx *c, long long *nodes, int *q, int *slot_byt
     return LBMC_OK;
 }
 
+lbmc_status lbmc_pass_info(lbmc_ctx *c, int *calls, int *width, int *height)
+{
+    if (!c) return fail(nullptr, LBMC_ERR_INVALID, "null context");
+    std::lock_guard<std::mutex> lock(c->pass_mu);
+    const bool on = c->tile.on;
+    if (calls) *calls = on ? c->tile.M + 1 : 1;
+    if (width) *width = on ? c->tile.W : 0;
+    if (height) *height = on ? c->tile.H : 0;
+    return LBMC_OK;
+}
+
 lbmc_status lbmc_copy_bandwidth(int device, size_t nbytes, int reps, float *ms)
 {
     if (!ms || nbytes == 0 || nbytes % 16 != 0 || reps <= 0)

@@ -34,7 +34,7 @@ STATUS = {0: "LBMC_OK", 1: "LBMC_ERR_INVALID", 2: "LBMC_ERR_NOMEM", 3: "LBMC_ERR
 EXPORTS = [
     "lbmc_create", "lbmc_destroy", "lbmc_last_error", "lbmc_set_fields", "lbmc_get_node_types",
     "lbmc_get_links", "lbmc_init_static", "lbmc_init_equilibrium", "lbmc_step", "lbmc_run",
-    "lbmc_time_steps", "lbmc_get_macros", "lbmc_get_node", "lbmc_get_f", "lbmc_set_f",
+    "lbmc_pass_info", "lbmc_time_steps", "lbmc_get_macros", "lbmc_get_node", "lbmc_get_f", "lbmc_set_f",
     "lbmc_get_f_noalloc",
     "lbmc_kinetic_energy", "lbmc_sync", "lbmc_info", "lbmc_copy_bandwidth",
     "lbmc_mlp_create", "lbmc_mlp_destroy", "lbmc_mlp_last_error", "lbmc_mlp_set_params",
@@ -98,6 +98,7 @@ def _load():
         "lbmc_init_equilibrium": (ct.c_int, [P, ct.POINTER(ct.c_double), dpp]),
         "lbmc_step": (ct.c_int, [P, ct.c_longlong, ct.c_int]),
         "lbmc_run": (ct.c_int, [P, ct.c_longlong, ct.c_int, ct.c_int]),
+        "lbmc_pass_info": (ct.c_int, [P] + [ct.POINTER(ct.c_int)] * 3),
         "lbmc_time_steps": (ct.c_int, [P, ct.c_longlong, ct.c_int, ct.c_int,
                                        ct.POINTER(ct.c_float)]),
         "lbmc_get_macros": (ct.c_int, [P, ct.POINTER(ct.c_double), dpp]),
@@ -274,6 +275,13 @@ class Lattice:
 
     def run(self, t0, nsteps, store_every=1):
         self._check(_lib.lbmc_run(self._h, int(t0), int(nsteps), int(store_every)))
+
+    def pass_info(self):
+        """Calls that run() takes per pass over memory (1: one per launch) and
+        the tile of a pass, margins included."""
+        v = [ct.c_int() for _ in range(3)]
+        self._check(_lib.lbmc_pass_info(self._h, *(ct.byref(k) for k in v)))
+        return {"calls": v[0].value, "width": v[1].value, "height": v[2].value}
 
     def time_steps(self, t0, nsteps, store_every=0):
         ms = ct.c_float()
