@@ -349,12 +349,18 @@ lbmc_status follow_closures(lbmc_batch *b)
 // ---- passes of several calls (D2Q9 members in 32 or 64 bits that all hold a
 // second population buffer)
 
-// tiles of every member, all of them with the margin of one pass length
+bool has_tiles(const lbmc_batch *b)
+{
+    return b->lattice == LBMC_D2Q9 && (b->storage == LBMC_FP64 || b->storage == LBMC_FP32);
+}
+
+// tiles of every member, all of them with the margin of one pass length.
+// Allocates, so no member's pass_mu is held (dev_malloc).
 lbmc_status build_tiles(lbmc_batch *b)
 {
     std::vector<char> closure;
     for (const lbmc_ctx *c : b->members) closure.push_back(c->key.closure ? 1 : 0);
-    if (b->tiles && closure == b->tile_closure) return LBMC_OK;
+    if (b->tiles && b->dpass && closure == b->tile_closure) return LBMC_OK;
     const int slot = (int)b->members[0]->sbytes;
     const TileCapacity cap = tile_capacity(2, slot);
     const int P = cap.threads * cap.per_thread;
@@ -407,7 +413,6 @@ lbmc_status build_tiles(lbmc_batch *b)
 // the closure members evaluate on the first call.
 bool can_pass(const lbmc_batch *b, long long t0, int store_every, int *every, bool *eval0)
 {
-    if (b->lattice != LBMC_D2Q9 || (b->storage != LBMC_FP64 && b->storage != LBMC_FP32)) return false;
     *every = 0;
     *eval0 = false;
     int seen = 0, ev = 0;
@@ -519,12 +524,13 @@ lbmc_status pass_steps(lbmc_batch *b, long long t0, int nsteps, int store_every,
 lbmc_status run_in_passes(lbmc_batch *b, long long t0, int nsteps, int store_every, bool timed, bool *done)
 {
     *done = false;
+    // no memory for the lists: one call per launch needs none
+    if (nsteps <= 0 || !has_tiles(b) || build_tiles(b) != LBMC_OK) return LBMC_OK;
     std::vector<std::unique_lock<std::mutex>> locks;
     for (lbmc_ctx *c : b->members) locks.emplace_back(c->pass_mu);
     int every = 0;
     bool eval0 = false;
-    if (nsteps <= 0 || !can_pass(b, t0, store_every, &every, &eval0)) return LBMC_OK;
-    if (lbmc_status st = build_tiles(b)) return st;
+    if (!can_pass(b, t0, store_every, &every, &eval0)) return LBMC_OK;
     if (b->ntiles_closure && (!b->mlp || !b->cchunks)) return LBMC_OK;
     *done = true;
     if (lbmc_status st = b->cdouble ? upload_pass_members<double>(b, t0) : upload_pass_members<float>(b, t0)) return st;
@@ -633,8 +639,7 @@ lbmc_status lbmc_batch_create(lbmc_ctx *const *members, int count, lbmc_batch **
     b->grid = (int)std::min<long long>(b->nchunks, 8LL * b->ncu);
     if (hipDeviceGetAttribute(&b->lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, b->device) != hipSuccess)
         b->lds_cu = 0;
-    if (b->lattice == LBMC_D2Q9 && (b->storage == LBMC_FP64 || b->storage == LBMC_FP32))
-        if (lbmc_status st = build_tiles(b)) return bail(st);
+    if (has_tiles(b)) (void)build_tiles(b);  // tried again by every run
     *out = b;
     return LBMC_OK;
 }

@@ -494,7 +494,9 @@ namespace lbmc {
 
 hipError_t dev_malloc(void **p, size_t bytes)
 {
-    hipError_t e = hipMalloc(p, bytes);
+    // test hook: LBMC_OOM=n: none for n bytes or more until a buffer was given back
+    const char *env = getenv("LBMC_OOM");
+    hipError_t e = env && bytes >= strtoull(env, nullptr, 10) ? hipErrorOutOfMemory : hipMalloc(p, bytes);
     if (e != hipErrorOutOfMemory) return e;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return e;
