@@ -64,8 +64,8 @@ struct lbmc_ctx {
 
     // passes of several calls (tile_kernel.hpp, march_kernel.hpp): tile shape, and the second
     // population buffer that they write to (null: one call per launch).
-    // pass_mu: held while launches that use f2 are issued, and by another
-    // thread that takes f2 back when device memory runs out (dev_malloc)
+    // pass_mu: held while a run's launches are issued or captured, and by
+    // another thread that takes f2 back when device memory runs out (dev_malloc)
     lbmc::TilePlan tile{};
     void *f2 = nullptr;
     long long npad2 = 0;  // elements between f2's direction arrays

@@ -440,12 +440,12 @@ lbmc_status run_steps(lbmc_ctx *c, long long t0, int nsteps, int store_every)
         t0++;
         nsteps--;
     }
-    {
-        std::lock_guard<std::mutex> lock(c->pass_mu);
-        if (c->tile.on && !c->key.closure) return run_in_passes(c, t0, nsteps, store_every);
-        // two calls between evaluations at least
-        if (c->tile.on && c->D == 3 && c->closure_every > 2) return run_closure_in_passes(c, t0, nsteps, store_every);
-    }
+    // also while a graph is captured: a thread that gives this lattice's second
+    // buffer back waits for the stream, which a capture does not allow
+    std::lock_guard<std::mutex> lock(c->pass_mu);
+    if (c->tile.on && !c->key.closure) return run_in_passes(c, t0, nsteps, store_every);
+    // two calls between evaluations at least
+    if (c->tile.on && c->D == 3 && c->closure_every > 2) return run_closure_in_passes(c, t0, nsteps, store_every);
     auto stores = [&](long long tt) { return store_every > 0 && ((tt + 1) % store_every) == 0; };
     long long period = lcm_ll(lcm_ll(c->L[0], c->L[1]), c->L[2]);
     if (store_every > 0) period = lcm_ll(period, store_every);

@@ -128,3 +128,51 @@ def test_given_back_while_others_run(monkeypatch):
         _same(_read(lat), want)
         lat.close()
     other.close()
+
+
+def test_given_back_while_a_graph_is_captured(monkeypatch):
+    # a closure lattice holds a buffer (for batches) and replays one call per
+    # launch from a captured graph, 2016 launches long here
+    case = cases.channel_d2q9(63, 32)
+    model = lbmc.Mlp(pymlp.flatten(pymlp.init_params(3)), mu=[0] * 6 + [1], isd=[300.0] * 6 + [100.0], out_a=0.02,
+                     out_b=0.8)
+
+    def built():
+        lat = cases.build(lbmc.Lattice, case, storage=1)
+        lat.set_closure(model, 0.6, 1.0)
+        return lat
+
+    plain = built()
+    for t in range(0, 4032, 7):
+        plain.run(t, 7, 0)
+    want = _read(plain)
+    plain.close()
+    other = cases.build(lbmc.Lattice, cases.sf_d2q9(), storage=1)
+    for _ in range(4):
+        lat, errors, begun, over = built(), [], threading.Event(), threading.Event()
+        assert _calls(lat) > 1
+
+        def work():
+            begun.set()
+            try:
+                lat.run(0, 4032, 0)
+            except BaseException as e:  # noqa: BLE001
+                errors.append(e)
+            over.set()
+
+        monkeypatch.setenv("LBMC_OOM", "1")
+        thread = threading.Thread(target=work)
+        thread.start()
+        begun.wait()
+        while not over.is_set():
+            try:
+                other.get_f()
+            except lbmc.LbmcError:
+                pass  # the buffer was in use, or was given back before
+        thread.join()
+        monkeypatch.delenv("LBMC_OOM")
+        assert not errors
+        _same(_read(lat), want)
+        lat.close()
+    other.close()
+    model.close()
