@@ -1198,8 +1198,8 @@ lbmc_status lbmc_copy_bandwidth(int device, size_t nbytes, int reps, float *ms)
     void *a = nullptr, *b = nullptr;
     hipStream_t s = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
-    e = hipMalloc(&a, nbytes);
-    if (e == hipSuccess) e = hipMalloc(&b, nbytes);
+    e = dev_malloc(&a, nbytes);
+    if (e == hipSuccess) e = dev_malloc(&b, nbytes);
     if (e == hipSuccess) e = hipMemset(a, 1, nbytes);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreate(&e0);

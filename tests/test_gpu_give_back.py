@@ -176,3 +176,17 @@ def test_given_back_while_a_graph_is_captured(monkeypatch):
         lat.close()
     other.close()
     model.close()
+
+
+def test_given_back_to_the_copy_measurement(monkeypatch):
+    lat = cases.build(lbmc.Lattice, cases.channel_d2q9(64, 48), storage=1)
+    small = cases.build(lbmc.Lattice, cases.channel_d2q9(32, 16), storage=1)
+    # 1 MB each: the first finds a buffer to give back
+    monkeypatch.setenv("LBMC_OOM", str(1 << 20))
+    with pytest.raises(lbmc.LbmcError):
+        lbmc.copy_bandwidth(1 << 20, 1)  # nothing left for the second
+    monkeypatch.delenv("LBMC_OOM")
+    assert _calls(lat) == _calls(small) == 1
+    assert lbmc.copy_bandwidth(1 << 20, 1) > 0
+    lat.close()
+    small.close()
