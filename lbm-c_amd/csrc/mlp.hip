@@ -415,6 +415,7 @@ lbmc_status ensure_partial(lbmc_mlp *m, int nw)
     if (nw <= m->pcap) return LBMC_OK;
     if (m->partial) MLP_HIP(m, hipFree(m->partial));
     m->partial = nullptr;
+    m->pcap = 0;  // should the allocation fail
     MLP_HIP(m, dev_malloc((void **)&m->partial, (size_t)nw * MLP_PSTRIDE * sizeof(float)));
     m->pcap = nw;
     return LBMC_OK;

@@ -190,3 +190,23 @@ def test_given_back_to_the_copy_measurement(monkeypatch):
     assert lbmc.copy_bandwidth(1 << 20, 1) > 0
     lat.close()
     small.close()
+
+
+def test_training_after_a_step_without_memory(monkeypatch):
+    rng = np.random.default_rng(4)
+    x, y = np.float32(rng.standard_normal((20000, 7))), np.float32(rng.standard_normal(20000))
+    out = []
+    for fails in (False, True):
+        model = lbmc.Mlp(pymlp.flatten(pymlp.init_params(3)))
+        model.set_data(x, y)
+        loss = [model.train(1, batch=64, seed=1)]
+        if fails:
+            monkeypatch.setenv("LBMC_OOM", "1")
+            with pytest.raises(lbmc.LbmcError):
+                model.train(1, batch=20000, seed=2)  # needs more gradient records
+            monkeypatch.delenv("LBMC_OOM")
+        loss.append(model.train(1, batch=64, seed=3))
+        loss.append(model.train(1, batch=20000, seed=4))
+        out.append([*loss, model.get_params()])
+        model.close()
+    _same(out[1], out[0])
