@@ -762,6 +762,7 @@ lbmc_status lbmc_set_fields(lbmc_ctx *c, const double *geometry, const int *macr
         maskv[(size_t)n] = (uint8_t)cls_of[descv[(size_t)n]];
         all_fluid = all_fluid && maskv[(size_t)n] == 0;
     }
+    c->fields_set = false;  // until all of them are: an array may find no memory
     c->all_fluid = all_fluid;
     {
         std::lock_guard<std::mutex> lock(c->pass_mu);

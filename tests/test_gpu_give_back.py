@@ -210,3 +210,25 @@ def test_training_after_a_step_without_memory(monkeypatch):
         out.append([*loss, model.get_params()])
         model.close()
     _same(out[1], out[0])
+
+
+def test_fields_without_memory_are_not_run(monkeypatch):
+    case = cases.porous_d2q9(L=40, collision=cases.NTPOR)
+    want = _alone(monkeypatch, case, 1, 20)
+    lat = cases.build(lbmc.Lattice, case, storage=1)
+    fields = case["fields"]
+    # fluid everywhere: no buffer to give back, no porosity array yet
+    monkeypatch.setenv("LBMC_PASS", "0")
+    lat.set_fields(geometry=np.zeros(lat.n), force=fields["force"])
+    monkeypatch.setenv("LBMC_OOM", "1")
+    with pytest.raises(lbmc.LbmcError):
+        lat.set_fields(**fields)
+    monkeypatch.delenv("LBMC_OOM")
+    for call in (lambda: lat.run(0, 5, 1), lambda: lat.step(0), lambda: lbmc.Batch([lat])):
+        with pytest.raises(lbmc.LbmcError) as e:
+            call()
+        assert e.value.status == 4  # no fields
+    lat.set_fields(**fields)
+    lat.run(0, 20, 3)
+    _same(_read(lat), want)
+    lat.close()
