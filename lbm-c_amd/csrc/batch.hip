@@ -68,6 +68,7 @@ struct lbmc_batch {
     long long nodes = 0;
     int grid = 1;
     int sub = 1;            // 256-node tiles per chunk
+    int csub = 1;           //   and per chunk of the closure members' list
     int blocks_per_cu = 0;  // residency cap of the step kernel (0: none)
     int lds = 0;            //   as dynamic LDS bytes per block
     int lds_cu = 0;         // LDS bytes per CU
@@ -164,7 +165,7 @@ lbmc_status launch_one_step(lbmc_batch *b, int j)
     const size_t msz = b->cdouble ? sizeof(BatchMember<double>) : sizeof(BatchMember<float>);
     const void *members = (const char *)b->dwindow + (size_t)j * (size_t)b->count * msz;
     const BatchShape sh{b->grid, b->sub, b->lds};
-    const BatchEval ev{b->cchunks, b->mlp ? b->ncchunks : 0, b->eval_grid, b->mlp, b->any_eval + j,
+    const BatchEval ev{b->cchunks, b->mlp ? b->ncchunks : 0, b->eval_grid, b->csub, b->mlp, b->any_eval + j,
                        b->closure_fp16 != 0};
     switch (b->storage) {
     case LBMC_FP64: e = launch_batch_fp64(b->lattice, members, b->chunks, b->nchunks, b->grid, b->sub, b->lds, b->stream); break;
@@ -301,9 +302,11 @@ lbmc_status build_closure_chunks(lbmc_batch *b, int sub)
     int2 *list;
     int count;
     if (lbmc_status st = upload_chunks(b, sub, true, &list, &count)) return st;
+    drop_batch_graph(b);  // captured with the old list
     if (b->cchunks) (void)hipFree(b->cchunks);
     b->cchunks = list;
     b->ncchunks = count;
+    b->csub = sub;
     b->chunk_closure.clear();
     for (const lbmc_ctx *c : b->members) b->chunk_closure.push_back(c->key.closure ? 1 : 0);
     // evaluation kernel: persistent, 4 blocks per CU (its residency)
@@ -341,9 +344,7 @@ lbmc_status follow_closures(lbmc_batch *b)
     }
     if (mlp != b->mlp) drop_batch_graph(b);
     b->mlp = mlp;
-    if (closure == b->chunk_closure) return LBMC_OK;
-    drop_batch_graph(b);
-    return build_closure_chunks(b, b->sub);
+    return closure == b->chunk_closure ? LBMC_OK : build_closure_chunks(b, b->csub);
 }
 
 // ---- passes of several calls (D2Q9 members in 32 or 64 bits that all hold a
@@ -504,7 +505,7 @@ lbmc_status pass_steps(lbmc_batch *b, long long t0, int nsteps, int store_every,
                 bp.offset = k;
                 bp.store = stores(k) ? 1u : 0u;
                 bp.odd = *odd_closure;
-                const hipError_t err = launch_batch_call_fp32(b->dpass, b->cchunks, b->ncchunks, b->eval_grid, b->sub,
+                const hipError_t err = launch_batch_call_fp32(b->dpass, b->cchunks, b->ncchunks, b->eval_grid, b->csub,
                                                               b->mlp, every > 1, b->closure_fp16 != 0, bp, b->stream);
                 if (err != hipSuccess)
                     return bfail(b, LBMC_ERR_DEVICE, "batch call launch: %s", hipGetErrorString(err));
@@ -555,6 +556,27 @@ void mark_records(lbmc_batch *b)
 lbmc_status sync_members(lbmc_batch *b)
 {
     for (lbmc_ctx *c : b->members) B_HIP(b, hipStreamSynchronize(c->stream));
+    return LBMC_OK;
+}
+
+// lbmc_batch_time_steps; passes false: one call per launch
+lbmc_status time_calls(lbmc_batch *b, long long t0, int nsteps, int store_every, bool passes, float *ms)
+{
+    lbmc_status st = sync_members(b);
+    if (st == LBMC_OK) st = follow_closures(b);
+    bool done = false;
+    if (st == LBMC_OK && passes) st = run_in_passes(b, t0, nsteps, store_every, true, &done);
+    if (st == LBMC_OK && !done) st = upload(b, t0, store_every);  // outside the timed region
+    if (st != LBMC_OK) return st;
+    if (!done) {
+        B_HIP(b, hipEventRecord(b->ev0, b->stream));
+        st = batch_steps(b, t0, nsteps);
+        if (st != LBMC_OK) return st;
+        B_HIP(b, hipEventRecord(b->ev1, b->stream));
+    }
+    mark_records(b);
+    B_HIP(b, hipEventSynchronize(b->ev1));
+    B_HIP(b, hipEventElapsedTime(ms, b->ev0, b->ev1));
     return LBMC_OK;
 }
 
@@ -684,22 +706,7 @@ lbmc_status lbmc_batch_time_steps(lbmc_batch *b, long long t0, int nsteps, int s
 {
     if (!b || nsteps <= 0 || t0 < 0 || !ms) return bfail(b, LBMC_ERR_INVALID, "lbmc_batch_time_steps: bad argument");
     B_HIP(b, hipSetDevice(b->device));
-    lbmc_status st = sync_members(b);
-    if (st == LBMC_OK) st = follow_closures(b);
-    bool done = false;
-    if (st == LBMC_OK) st = run_in_passes(b, t0, nsteps, store_every, true, &done);
-    if (st == LBMC_OK && !done) st = upload(b, t0, store_every);  // outside the timed region
-    if (st != LBMC_OK) return st;
-    if (!done) {
-        B_HIP(b, hipEventRecord(b->ev0, b->stream));
-        st = batch_steps(b, t0, nsteps);
-        if (st != LBMC_OK) return st;
-        B_HIP(b, hipEventRecord(b->ev1, b->stream));
-    }
-    mark_records(b);
-    B_HIP(b, hipEventSynchronize(b->ev1));
-    B_HIP(b, hipEventElapsedTime(ms, b->ev0, b->ev1));
-    return LBMC_OK;
+    return time_calls(b, t0, nsteps, store_every, true, ms);
 }
 
 // Residency cap of the batch step kernel: at most `per` blocks per CU,
@@ -714,8 +721,14 @@ void set_blocks_per_cu(lbmc_batch *b, int per)
 // Times candidate launch shapes over a few steps from the current state and
 // keeps the fastest: chunks of 1, 2, 4 or 8 tiles with one block per chunk
 // and the resident blocks per CU uncapped or capped at 4 or 6, and
-// persistent grids of 2, 4, 8, 16 blocks per CU over one-tile chunks.  The
-// steps advance the members' state; callers tune before the timed run.
+// persistent grids of 2, 4, 8, 16 blocks per CU over one-tile chunks.  These
+// are shapes of the one-call launches, so the trials make one call per launch
+// also where runs go in passes: the shape then serves the runs that cannot
+// (16 members of 64 x 48: 4.6 us per call with 256-node chunks, 12.4 with
+// 2048).  Of a pass only the evaluating calls have chunks, the closure members'
+// own; they are timed in runs as they go (64 channels, network every call: 245
+// us per call with 256-node chunks, 231 with 2048).  The steps advance the
+// members' state; callers tune before the timed run.
 lbmc_status lbmc_batch_autotune(lbmc_batch *b, long long t0, int steps_per_trial, int *grid, float *ms_per_step)
 {
     if (!b || steps_per_trial <= 0 || t0 < 0) return bfail(b, LBMC_ERR_INVALID, "lbmc_batch_autotune: bad argument");
@@ -732,21 +745,21 @@ lbmc_status lbmc_batch_autotune(lbmc_batch *b, long long t0, int steps_per_trial
     Cand best_c{b->sub, 0, b->blocks_per_cu};
     int best_grid = b->grid;
     long long t = t0;
+    // one untimed pass (graph build), then the timed one
+    auto trial = [&](bool passes, float *ms) -> lbmc_status {
+        for (int k = 0; k < 2; k++, t += steps_per_trial)
+            if (lbmc_status st = time_calls(b, t, steps_per_trial, 0, passes, ms)) return st;
+        return LBMC_OK;
+    };
     for (const Cand &cd : cand) {
         set_blocks_per_cu(b, cd.cap);
         if (cd.cap && !b->blocks_per_cu) continue;  // cap not available
         drop_batch_graph(b);
-        if (cd.sub != b->sub)
+        if (cd.sub != b->sub || cd.sub != b->csub)
             if (lbmc_status st = build_chunks(b, cd.sub)) return st;
         b->grid = cd.grid_per_cu ? (int)std::min<long long>(b->nchunks, (long long)cd.grid_per_cu * ncu) : b->nchunks;
         float ms = 0.f;
-        // one untimed pass (graph build), then the timed one
-        lbmc_status st = lbmc_batch_time_steps(b, t, steps_per_trial, 0, &ms);
-        if (st != LBMC_OK) return st;
-        t += steps_per_trial;
-        st = lbmc_batch_time_steps(b, t, steps_per_trial, 0, &ms);
-        if (st != LBMC_OK) return st;
-        t += steps_per_trial;
+        if (lbmc_status st = trial(false, &ms)) return st;
         if (best < 0.f || ms < best) {
             best = ms;
             best_c = cd;
@@ -755,10 +768,35 @@ lbmc_status lbmc_batch_autotune(lbmc_batch *b, long long t0, int steps_per_trial
         }
     }
     drop_batch_graph(b);
-    if (best_c.sub != b->sub)
+    if (best_c.sub != b->sub || best_c.sub != b->csub)
         if (lbmc_status st = build_chunks(b, best_c.sub)) return st;
     b->grid = std::min(best_grid, b->nchunks);
     set_blocks_per_cu(b, best_c.cap);
+    // runs in passes: their evaluating calls' chunks, and their time per step
+    int every = 0;
+    bool eval0 = false, passes = has_tiles(b) && b->tiles;
+    if (passes) {
+        std::vector<std::unique_lock<std::mutex>> locks;
+        for (lbmc_ctx *c : b->members) locks.emplace_back(c->pass_mu);
+        passes = can_pass(b, t, 0, &every, &eval0);
+    }
+    if (passes) {
+        best = -1.f;
+        int best_sub = b->csub;
+        for (int sub : {1, 2, 4, 8}) {
+            if (b->ncchunks && sub != b->csub)
+                if (lbmc_status st = build_closure_chunks(b, sub)) return st;
+            float ms = 0.f;
+            if (lbmc_status st = trial(true, &ms)) return st;
+            if (best < 0.f || ms < best) {
+                best = ms;
+                best_sub = b->csub;
+            }
+            if (!b->ncchunks) break;  // nothing to choose
+        }
+        if (best_sub != b->csub)
+            if (lbmc_status st = build_closure_chunks(b, best_sub)) return st;
+    }
     if (grid) *grid = b->grid;
     if (ms_per_step) *ms_per_step = best / (float)steps_per_trial;
     return LBMC_OK;
@@ -784,7 +822,7 @@ lbmc_status lbmc_batch_set_shape(lbmc_batch *b, int grid, int chunk_nodes, int b
                      "lbmc_batch_set_shape: grid > 0, chunk_nodes a multiple of 256 up to 16384, blocks_per_cu >= 0");
     B_HIP(b, hipSetDevice(b->device));
     drop_batch_graph(b);
-    if (chunk_nodes / kBlock != b->sub)
+    if (chunk_nodes / kBlock != b->sub || chunk_nodes / kBlock != b->csub)
         if (lbmc_status st = build_chunks(b, chunk_nodes / kBlock)) return st;
     b->grid = std::min(grid, b->nchunks);
     set_blocks_per_cu(b, blocks_per_cu);

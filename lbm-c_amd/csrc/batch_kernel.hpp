@@ -237,11 +237,11 @@ struct BatchShape {
 };
 
 // The closure members' evaluation: their chunk list (nchunks 0: no closure
-// members), its grid, the shared weights, the device flag and the operand
+// members), its grid and tiles per chunk, the shared weights, the device flag and the operand
 // precision (fp16: true, else bf16)
 struct BatchEval {
     const int2 *chunks;
-    int nchunks, grid;
+    int nchunks, grid, sub;
     const void *mlp;
     const int *any_eval;
     bool fp16;
@@ -258,11 +258,11 @@ hipError_t launch_batch_lattice(const void *members, const int2 *chunks, int nch
         if (ev.nchunks > 0) {
             if (ev.fp16)
                 hipLaunchKernelGGL((batch_eval_kernel<L, St, true>), dim3(ev.grid), dim3(kBlock), 0, s,
-                                   (const BatchMember<float> *)members, ev.chunks, ev.nchunks, ev.mlp, sh.sub,
+                                   (const BatchMember<float> *)members, ev.chunks, ev.nchunks, ev.mlp, ev.sub,
                                    ev.any_eval);
             else
                 hipLaunchKernelGGL((batch_eval_kernel<L, St, false>), dim3(ev.grid), dim3(kBlock), 0, s,
-                                   (const BatchMember<float> *)members, ev.chunks, ev.nchunks, ev.mlp, sh.sub,
+                                   (const BatchMember<float> *)members, ev.chunks, ev.nchunks, ev.mlp, ev.sub,
                                    ev.any_eval);
         }
     }
