@@ -67,6 +67,7 @@ struct lbmc_ctx {
     // pass_mu: held while a run's launches are issued or captured, and by
     // another thread that takes f2 back when device memory runs out (dev_malloc)
     lbmc::TilePlan tile{};
+    lbmc::TilePlan tile_of[lbmc::kMaxPassCalls + 1]{};  // D2Q9: the tiles of a pass of k calls
     void *f2 = nullptr;
     long long npad2 = 0;  // elements between f2's direction arrays
     int march_cls = 0;  // node classes of a D3Q15 lattice's passes (MARCH_*)

@@ -227,11 +227,14 @@ void plan_passes(lbmc_ctx *c)
     } else if (c->D == 2 && !c->offsets64) {
         if (!env) {
             q = plan_tiles(c->L[0], c->L[1], slot, ncu, plain);
-        } else if (nv == 4 && v[0] >= 0 && v[0] <= 2 && v[3] < 32) {
+            for (int k = 2; q.on && k <= q.M; k++) c->tile_of[k] = plan_short(q, c->L[0], c->L[1], slot, ncu, plain, k);
+        } else if (nv == 4 && v[0] >= 0 && v[0] <= 2 && v[3] < kMaxPassCalls) {
             const TileCapacity cap = tile_capacity(v[0], slot);
             q.on = (long long)v[1] * v[2] <= cap.threads * cap.per_thread &&
                    tile_shape(c->L[0], c->L[1], v[0], v[1], v[2], v[3], q);
+            for (int k = 2; q.on && k <= q.M; k++) tile_shape(c->L[0], c->L[1], v[0], v[1], v[2], k - 1, c->tile_of[k]);
         }
+        if (q.on) c->tile_of[q.M + 1] = q;
     } else if (c->D == 3 && slot >= 4 && march_takes(slot, c->key.family != 0, c->key.mfix != 0, c->key.guo != 0) &&
                (unsigned long long)c->L[0] * c->L[1] * slot < (1ULL << 31)) {
         c->march_cls = c->all_fluid ? MARCH_FLUID : MARCH_SOLID;
@@ -320,9 +323,10 @@ hipError_t launch_pass(lbmc_ctx *c, long long t, int calls, unsigned store, bool
         if constexpr (sizeof(C) == 8) return launch_march_fp64(c->key, a, p, c->stream);
         else return launch_march_fp32(c->key, a, p, c->stream);
     }
+    const TilePlan &q = c->tile_of[calls];
     TilePass p;
     memset(&p, 0, sizeof(p));
-    tile_geometry(c->tile, c->L, p);
+    tile_geometry(q, c->L, p);
     p.src = src;
     p.dst = dst;
     p.calls = calls;
@@ -332,26 +336,26 @@ hipError_t launch_pass(lbmc_ctx *c, long long t, int calls, unsigned store, bool
         p.rs[d] = first ? a.s[d] : 1 % c->L[d];
         p.ws[d] = last ? (int)((t + calls - 1) % c->L[d]) : 0;
     }
-    const int tiles = c->tile.ntx * c->tile.nty;
+    const int tiles = q.ntx * q.nty;
     if constexpr (sizeof(C) == 8) {
-        return launch_tile_fp64(c->key, c->tile.size, a, p, tiles, c->stream);
+        return launch_tile_fp64(c->key, q.size, a, p, tiles, c->stream);
     } else {
         switch (c->storage) {
-        case LBMC_FP32: return launch_tile_fp32(c->key, c->tile.size, a, p, tiles, c->stream);
-        case LBMC_FP16S: return launch_tile_fp16s(c->key, c->tile.size, a, p, tiles, c->stream);
-        default: return launch_tile_bf16s(c->key, c->tile.size, a, p, tiles, c->stream);
+        case LBMC_FP32: return launch_tile_fp32(c->key, q.size, a, p, tiles, c->stream);
+        case LBMC_FP16S: return launch_tile_fp16s(c->key, q.size, a, p, tiles, c->stream);
+        default: return launch_tile_bf16s(c->key, q.size, a, p, tiles, c->stream);
         }
     }
 }
 
-// len >= 2 calls from t: an even number of passes, so that the state ends in
-// the buffer it started in.  D2Q9 passes share the calls out evenly; D3Q15
-// passes take two each, and the last up to three calls run one by one.
+// len calls from t: an even number of passes, so that the state ends in the
+// buffer it started in (tile_passes; D3Q15 passes take two calls each), and
+// the last up to three calls one by one.
 lbmc_status run_passes(lbmc_ctx *c, long long t, long long len, int store_every)
 {
     const int K = c->tile.M + 1;
-    const long long np = c->D == 2 ? 2 * ((len + 2 * K - 1) / (2 * K)) : 2 * (len / (2 * K));
-    long long rest = c->D == 2 ? 0 : len - K * np;
+    const long long np = c->D == 2 ? tile_passes(len, K) : 2 * (len / (2 * K));
+    long long rest = std::max(0LL, len - K * np);
     len -= rest;
     for (long long k = 0; k < np; k++) {
         const long long k0 = len * k / np, k1 = len * (k + 1) / np;
@@ -379,7 +383,7 @@ lbmc_status run_in_passes(lbmc_ctx *c, long long t, int nsteps, int store_every)
     while (t < end) {
         long long e = end;
         if (c->has_macro && store_every > 0) e = std::min(end, (t + store_every) / store_every * store_every - 1);
-        if (e - t >= 2) {
+        if (e > t) {
             if (lbmc_status st = run_passes(c, t, e - t, store_every)) return st;
             t = e;
         } else {
@@ -443,7 +447,9 @@ lbmc_status run_steps(lbmc_ctx *c, long long t0, int nsteps, int store_every)
     // also while a graph is captured: a thread that gives this lattice's second
     // buffer back waits for the stream, which a capture does not allow
     std::lock_guard<std::mutex> lock(c->pass_mu);
-    if (c->tile.on && !c->key.closure) return run_in_passes(c, t0, nsteps, store_every);
+    // calls between those that run alone (run_in_passes)
+    const int stretch = c->has_macro && store_every > 0 ? std::min(nsteps, store_every - 1) : nsteps;
+    if (c->tile.on && !c->key.closure && stretch >= kMinPassRun) return run_in_passes(c, t0, nsteps, store_every);
     // two calls between evaluations at least
     if (c->tile.on && c->D == 3 && c->closure_every > 2) return run_closure_in_passes(c, t0, nsteps, store_every);
     auto stores = [&](long long tt) { return store_every > 0 && ((tt + 1) % store_every) == 0; };

@@ -10,6 +10,8 @@
 
 namespace lbmc {
 
+constexpr int kMaxPassCalls = 32;  // the bits of TilePass::store
+
 struct TilePass {
     const void *src;
     void *dst;
@@ -96,6 +98,37 @@ inline bool tile_shape(int Lx, int Ly, int size, int W, int H, int M, TilePlan &
     return true;
 }
 
+// Runs of fewer calls go one call per launch (us for 3 calls, one by one and in
+// passes of one and two: 2048 x 1024 FP64 143, 185, FP32 76, 86; 1148 x 450
+// FP16S 29, 40); with 4 passes are ahead in every format and size that has them
+// (1.04 to 1.8 times).
+constexpr int kMinPassRun = 4;
+
+// Passes of a run of len calls, K at most in each: an even number, so that the
+// state ends in the buffer it started in, of two calls or more each (a pass
+// of one call moves what a launch in place moves).  They share out min(len,
+// passes * K) calls evenly; the rest, up to three, go one by one.
+inline long long tile_passes(long long len, int K)
+{
+    const long long np = 2 * ((len + 2 * K - 1) / (2 * K));
+    return len < 2 * np ? np - 2 : np;
+}
+
+// ns of a CU per node update (tile_estimate)
+inline double tile_ns(int slot_bytes) { return slot_bytes == 8 ? 2.9 : slot_bytes == 4 ? 1.2 : 1.7; }
+
+// node updates of one tile in a pass, and its bytes
+inline double tile_updates(const TilePlan &q, int calls)
+{
+    double nodes = (double)q.OW * q.OH;
+    for (int j = 0; j + 1 < calls; j++) nodes += (double)(q.W - 2 * j) * (q.H - 2 * j);
+    return nodes;
+}
+inline double tile_bytes(const TilePlan &q, int slot_bytes)
+{
+    return 9 * (q.H * ((double)q.W * slot_bytes + 96) + q.OH * ((double)q.OW * slot_bytes + 96));
+}
+
 // Estimated time per call (us) of the passes of a plan.  Measured constants
 // (MI355X): 3.5 us for a launch with its first loads and last stores; per
 // call of a tile at least the latency of one update (0.5 us, 0.8 us in 64
@@ -103,18 +136,14 @@ inline bool tile_shape(int Lx, int Ly, int size, int W, int H, int M, TilePlan &
 // bits, which also round and convert); 20 bytes per ns and CU of memory
 // traffic, about half of it hidden under the arithmetic of the other
 // resident blocks.
-inline double tile_estimate(const TilePlan &q, int slot_bytes, int ncu)
+// calls: of a pass of fewer calls than the plan's M + 1.
+inline double tile_estimate(const TilePlan &q, int slot_bytes, int ncu, int calls)
 {
-    const double ns_node = slot_bytes == 8 ? 2.9 : slot_bytes == 4 ? 1.2 : 1.7;
     const double us_call = slot_bytes == 8 ? 0.8 : 0.5;
-    double nodes = 0;
-    for (int j = 0; j <= q.M; j++) nodes += (double)(q.W - 2 * j) * (q.H - 2 * j);
-    const double tiles = (double)q.ntx * q.nty;
-    double per_cu = tiles / ncu;
+    double per_cu = (double)q.ntx * q.nty / ncu;
     if (per_cu < 4) per_cu = std::max(1.0, (double)((long long)(per_cu + 0.999)));
-    const double arith = std::max((q.M + 1) * us_call, per_cu * nodes * ns_node * 1e-3);
-    const double bytes = per_cu * 9 * (q.H * ((double)q.W * slot_bytes + 96) + q.OH * ((double)q.OW * slot_bytes + 96));
-    return (3.5 + arith + 0.5 * bytes / 20e3) / (q.M + 1);
+    const double arith = std::max(calls * us_call, per_cu * tile_updates(q, calls) * tile_ns(slot_bytes) * 1e-3);
+    return (3.5 + arith + 0.5 * per_cu * tile_bytes(q, slot_bytes) / 20e3) / calls;
 }
 
 // The plan with the smallest estimate (within 10 % of the best of all
@@ -134,7 +163,8 @@ inline double tile_estimate(const TilePlan &q, int slot_bytes, int ncu)
 // 1222 x 1000 15.4 -> 13.4, 1400 x 1400 19.6 against 19.0-19.9; FP16S 800 x 640
 // 14.6 -> 8.4, one call per launch 11.9; 64 bits hold 1024 and gain 0-5 %).
 // M up to 7: deeper passes of the small tiles recompute more than they save.
-inline TilePlan plan_tiles(int Lx, int Ly, int slot_bytes, int ncu, bool plain)
+// calls: the plan for passes of that many (0: the best of all).
+inline TilePlan plan_tiles(int Lx, int Ly, int slot_bytes, int ncu, bool plain, int calls = 0)
 {
     TilePlan best;
     const long long nodes = (long long)Lx * Ly;
@@ -144,10 +174,10 @@ inline TilePlan plan_tiles(int Lx, int Ly, int slot_bytes, int ncu, bool plain)
         const TileCapacity cap = tile_capacity(size, slot_bytes);
         const int P = cap.threads * cap.per_thread;
         for (int W = 16; W <= 128; W *= 2)
-            for (int M = 1; M <= 7; M++) {
+            for (int M = calls ? calls - 1 : 1; M <= (calls ? calls - 1 : 7); M++) {
                 TilePlan q;
                 if (P / W < 8 || !tile_shape(Lx, Ly, size, W, P / W, M, q)) continue;
-                q.us = tile_estimate(q, slot_bytes, ncu);
+                q.us = tile_estimate(q, slot_bytes, ncu, M + 1);
                 q.on = true;
                 if (!best.on || q.us < best.us) best = q;
             }
@@ -155,15 +185,24 @@ inline TilePlan plan_tiles(int Lx, int Ly, int slot_bytes, int ncu, bool plain)
     return best;
 }
 
+// Tiles of a pass of fewer calls than the lattice's plan q has: q's, or others
+// with the margin that these calls need where they are estimated 10 % ahead, 5
+// % in 16 bits (below that the planned ones were up to 15 % ahead at 600 x 300,
+// 64 x 48).  Runs of 4 calls, us, one call per launch, q's tiles, these: FP32
+// 600 x 300 24.7, 26.3, 18.6; 2048 x 1024 102, 99, 76; FP64 2048 x 1024 190,
+// 203, 173; FP16S 1148 x 450 40, 48, 30.
+inline TilePlan plan_short(const TilePlan &q, int Lx, int Ly, int slot_bytes, int ncu, bool plain, int calls)
+{
+    const TilePlan s = plan_tiles(Lx, Ly, slot_bytes, ncu, plain, calls);
+    return s.on && s.us < (slot_bytes == 2 ? 0.95 : 0.9) * tile_estimate(q, slot_bytes, ncu, calls) ? s : q;
+}
+
 // Work of a plan's tiles per call, in ns of one CU (tile_estimate's terms),
 // for batches, whose tiles of all members fill the chip together.
 inline double tile_work(const TilePlan &q, int slot_bytes)
 {
-    const double ns_node = slot_bytes == 8 ? 2.9 : slot_bytes == 4 ? 1.2 : 1.7;
-    double nodes = 0;
-    for (int j = 0; j <= q.M; j++) nodes += (double)(q.W - 2 * j) * (q.H - 2 * j);
-    const double bytes = 9 * (q.H * ((double)q.W * slot_bytes + 96) + q.OH * ((double)q.OW * slot_bytes + 96));
-    return (double)q.ntx * q.nty * (nodes * ns_node + 0.5 * bytes / 20) / (q.M + 1);
+    return (double)q.ntx * q.nty *
+           (tile_updates(q, q.M + 1) * tile_ns(slot_bytes) + 0.5 * tile_bytes(q, slot_bytes) / 20) / (q.M + 1);
 }
 
 // the geometry half of a pass's arguments

@@ -91,3 +91,28 @@ def test_members_of_a_batch_hold_their_buffers(monkeypatch):
             assert _calls(lat) > 1
             batch.close()
             lat.close()
+
+
+@pytest.mark.parametrize("storage", [0, 1, 2, 3], ids=["f64", "f32", "f16s", "bf16s"])
+@pytest.mark.parametrize("case", [cases.channel_d2q9(300, 200), cases.pressure_d2q9(Lx=300, Ly=200),
+                                  cases.channel_d2q9(1148, 450), cases.pressure_d2q9(Lx=61, Ly=47)],
+                         ids=lambda c: c["name"])
+def test_runs_of_every_length(monkeypatch, case, storage):
+    """Every number of calls around the lengths of a pass, with the tiles of
+    each, and stretches of every length between stored prescribed values."""
+    out = []
+    for shape in ("0", None):
+        lat = _built(monkeypatch, case, storage, shape)
+        assert (_calls(lat) == 1) == (shape == "0")
+        t = 0
+        for n in range(1, 19):
+            lat.run(t, n, 0)
+            t += n
+        for store_every in range(1, 11):
+            lat.run(t, 23, store_every)
+            t += 23
+        rho, u = lat.get_macros()
+        out.append((lat.get_f(), rho, u))
+        lat.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
