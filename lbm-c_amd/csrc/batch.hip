@@ -409,18 +409,18 @@ lbmc_status build_tiles(lbmc_batch *b)
     return LBMC_OK;
 }
 
-// Whether a run from call t0 can go in passes: every member with a second
+// Whether a run from call t0 goes in passes: it pays, every member with a second
 // buffer (their pass_mu held), and closure members on one schedule.  *eval0:
 // the closure members evaluate on the first call.
-bool can_pass(const lbmc_batch *b, long long t0, int store_every, int *every, bool *eval0)
+bool can_pass(const lbmc_batch *b, long long t0, int nsteps, int store_every, int *every, bool *eval0)
 {
     *every = 0;
     *eval0 = false;
     int seen = 0, ev = 0;
+    bool macro = false;
     for (const lbmc_ctx *c : b->members) {
         if (!c->f2 || !c->tile.on || c->nsf || !c->fields_set || c->L[0] >= (1 << 30) || c->L[1] >= (1 << 30)) return false;
-        // every few calls alone: one call per launch in place moves less
-        if (c->has_macro && store_every > 0 && store_every < 4) return false;
+        macro = macro || c->has_macro;
         if (!c->key.closure) continue;
         if (*every && c->closure_every != *every) return false;
         *every = c->closure_every;
@@ -429,7 +429,8 @@ bool can_pass(const lbmc_batch *b, long long t0, int store_every, int *every, bo
     }
     if (ev != 0 && ev != seen) return false;
     *eval0 = ev != 0;
-    return true;
+    return batch_passes(BatchRun{b->nodes, (int)b->members[0]->sbytes, nsteps, store_every, macro, *every,
+                                 seen > 0 && seen < b->count});
 }
 
 template <class C>
@@ -531,7 +532,7 @@ lbmc_status run_in_passes(lbmc_batch *b, long long t0, int nsteps, int store_eve
     for (lbmc_ctx *c : b->members) locks.emplace_back(c->pass_mu);
     int every = 0;
     bool eval0 = false;
-    if (!can_pass(b, t0, store_every, &every, &eval0)) return LBMC_OK;
+    if (!can_pass(b, t0, nsteps, store_every, &every, &eval0)) return LBMC_OK;
     if (b->ntiles_closure && (!b->mlp || !b->cchunks)) return LBMC_OK;
     *done = true;
     if (lbmc_status st = b->cdouble ? upload_pass_members<double>(b, t0) : upload_pass_members<float>(b, t0)) return st;
@@ -778,7 +779,7 @@ lbmc_status lbmc_batch_autotune(lbmc_batch *b, long long t0, int steps_per_trial
     if (passes) {
         std::vector<std::unique_lock<std::mutex>> locks;
         for (lbmc_ctx *c : b->members) locks.emplace_back(c->pass_mu);
-        passes = can_pass(b, t, 0, &every, &eval0);
+        passes = can_pass(b, t, steps_per_trial, 0, &every, &eval0);
     }
     if (passes) {
         best = -1.f;

@@ -205,6 +205,48 @@ inline double tile_work(const TilePlan &q, int slot_bytes)
            (tile_updates(q, q.M + 1) * tile_ns(slot_bytes) + 0.5 * tile_bytes(q, slot_bytes) / 20) / (q.M + 1);
 }
 
+// A batch's run, for batch_passes
+struct BatchRun {
+    long long nodes;   // of all members
+    int slot_bytes;
+    int nsteps;
+    int store_every;
+    bool macro;        // some members prescribe values: the calls that store them run alone
+    int every;         // closure members' interval (0: none)
+    bool mixed;        // closure members and others, which go in launches of their own
+};
+
+// Whether a batch's run pays in passes.  Measured on D2Q9 batches of 4 to 128
+// members, 4600 to 6.7 M nodes, us per call in place -> in passes (runs of up
+// to 8 calls: per run, which upload less and gain 5-15 us by that).  Not
+// - one call, from 8 MB of slots per direction on, which saves no traffic: 6.7
+//   M nodes FP32 155 -> 193, FP64 244 -> 317; 2.1 M FP32 95 -> 95;
+// - prescribed values stored more often than every 4th call.
+// The rest in 32 bits only: tiles of 2048 nodes, four to a thread, make a small
+// batch wait for each call (tiles of 1024 in 64 bits are ahead: 16 x 96 x 64
+// between pressure faces 7.0 -> 5.5).  Not
+// - prescribed values below 2^19 nodes (MRT between pressure faces 16 x 96 x 64
+//   6.1 -> 6.9, 8 x 256 x 128 7.8 -> 8.3, 128 x 96 x 64 15.7 -> 15.1), stored now
+//   and then below 2^20 (every 12th call 128 x 96 x 64 15.6 -> 17.6, 64 x 256 x 128
+//   35 -> 30), every 4th to 6th below 2^22 (64 x 256 x 128 35.3 -> 36.5);
+// - the closure every 2nd call, a pass of one call each: 24 x 256 x 128 25.3 ->
+//   28.3; beside other members from 2^20 nodes on 28.0 -> 26.2 (4 x 701 x 397);
+// - the closure beside other members below 5 * 2^16 nodes, two lists of tiles
+//   that each leave part of the chip idle: 8 x 256 x 128, interval 8, 9.0 -> 10.8;
+//   64 x 96 x 64 12.0 -> 10.9.
+inline bool batch_passes(const BatchRun &r)
+{
+    if (r.nsteps == 1 && r.nodes * r.slot_bytes > (8LL << 20)) return false;
+    const bool stores = r.macro && r.store_every > 0;
+    if (stores && r.store_every < 4) return false;
+    if (r.slot_bytes != 4) return true;
+    if (stores && r.nodes < (r.store_every < 7 ? 1LL << 22 : 1LL << 20)) return false;
+    if (r.nsteps <= 8) return true;
+    if (r.macro && r.nodes < (1LL << 19)) return false;
+    if (r.every == 2) return r.mixed && r.nodes >= (1LL << 20);
+    return !(r.every > 2 && r.mixed && r.nodes < (5LL << 16));
+}
+
 // the geometry half of a pass's arguments
 inline void tile_geometry(const TilePlan &q, const int *L, TilePass &p)
 {

@@ -48,11 +48,49 @@ void tiles(int Lx, int Ly, int slot, bool plain)
     }
 }
 
+// batch_passes at both sides of each of its lines
+void batches()
+{
+    const long long M = 1LL << 20;
+    int n = 0;
+    auto expect = [&](bool want, const BatchRun &r) { check(batch_passes(r) == want, "batch", n++, r.nodes, r.nsteps); };
+    // one call
+    expect(true, {2 * M, 4, 1, 0, false, 0, false});
+    expect(false, {2 * M + 1, 4, 1, 0, false, 0, false});
+    expect(false, {M + 1, 8, 1, 0, false, 0, false});
+    expect(true, {1LL << 40, 8, 2, 1, false, 0, false});
+    // prescribed values
+    for (int nsteps : {2, 100})
+        for (int se : {1, 2, 3}) {
+            expect(false, {8 * M, 4, nsteps, se, true, 0, false});
+            expect(false, {8 * M, 8, nsteps, se, true, 0, false});
+        }
+    expect(true, {1, 8, 100, 4, true, 0, false});
+    expect(true, {1, 4, 8, 0, true, 0, false});
+    expect(false, {M / 2 - 1, 4, 9, 0, true, 0, false});
+    expect(true, {M / 2, 4, 9, 0, true, 0, false});
+    expect(false, {M - 1, 4, 9, 7, true, 0, false});
+    expect(true, {M, 4, 9, 7, true, 0, false});
+    expect(false, {4 * M - 1, 4, 2, 4, true, 0, false});
+    expect(true, {4 * M, 4, 2, 4, true, 0, false});
+    expect(true, {1, 4, 100, 1, false, 0, false});
+    // closure members
+    expect(true, {1, 4, 100, 0, false, 1, true});
+    expect(true, {1, 4, 8, 0, false, 2, false});
+    expect(false, {8 * M, 4, 9, 0, false, 2, false});
+    expect(false, {M - 1, 4, 9, 0, false, 2, true});
+    expect(true, {M, 4, 9, 0, false, 2, true});
+    expect(true, {1, 4, 9, 0, false, 3, false});
+    expect(false, {(5LL << 16) - 1, 4, 9, 0, false, 3, true});
+    expect(true, {5LL << 16, 4, 9, 0, false, 3, true});
+}
+
 }  // namespace
 
 int main()
 {
     splits();
+    batches();
     const int L[][2] = {{1, 1},     {3, 5},     {1, 5000},   {64, 48},     {97, 61},     {300, 200},
                         {600, 300}, {900, 500}, {1148, 450}, {1031, 1021}, {2048, 1024}, {3392, 3392}};
     for (const auto &l : L)

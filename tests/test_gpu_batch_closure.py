@@ -68,8 +68,10 @@ def test_closure_switched_between_runs(monkeypatch, storage, path, every):
     else:
         monkeypatch.setenv("LBMC_PASS", path)
     # 75 calls: the captured graph of the one-call path, before and after a
-    # change; then one member off, another on, all off, the first two on again
-    phases = [({}, 75), ({1: None, 2: every}, 75), ({0: None, 2: None}, 11), ({0: every, 1: every}, 9)]
+    # change; up to 8: passes; one member off, another on, all off, the first
+    # two on again
+    phases = [({}, 75), ({}, 8), ({1: None, 2: every}, 8), ({}, 75), ({0: None, 2: None}, 7), ({}, 11),
+              ({0: every, 1: every}, 8), ({}, 9)]
     want = _stepped(storage, {0: every, 1: every}, phases, False)
     got = _stepped(storage, {0: every, 1: every}, phases, True)
     for k, (g, w) in enumerate(zip(got, want)):
