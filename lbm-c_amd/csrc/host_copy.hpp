@@ -8,8 +8,9 @@
 
 namespace lbmc {
 
-// The process's staging memory (1 MB, and 16 MB more with the first larger
-// transfer): held by every context and every model, freed with the last.
+// The process's staging memory (1 MB with the first small transfer, 16 MB with
+// the first larger one): held by every context and every model, whose
+// transfers alone use it, freed with the last.
 void staging_hold();
 void staging_release();
 

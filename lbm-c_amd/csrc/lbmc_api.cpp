@@ -621,7 +621,7 @@ lbmc_status lbmc_create(const lbmc_desc *desc, lbmc_ctx **out)
         return st;
     };
     hipError_t e = hipSetDevice(desc->device);
-    staging_hold();  // on this device: a process that uses one touches no other
+    staging_hold();
     if (e != hipSuccess) return bail(hip_fail(c, e, "hipSetDevice"));
     if ((e = hipStreamCreate(&c->stream)) != hipSuccess)
         return bail(hip_fail(c, e, "hipStreamCreate"));
