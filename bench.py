@@ -38,17 +38,13 @@ sys.path.insert(0, os.path.join(ROOT, "lbm-c_amd"))
 HBM_PEAK_GBS = 8000.0  # MI355X HBM3E, vendor figure
 
 
-def step_bytes(slot_bytes, steps, L):
-    """Algorithmic bytes per node and step of an L^3 D3Q15 box: FP32 and FP64
-    runs take two calls per pass, in pairs of passes, and the rest one call
-    per launch; so do all calls of 16-bit lattices, of small ones and of FP64
-    ones that just fit the last-level cache (the library's plan_march)."""
+def step_bytes(slot_bytes, steps, calls):
+    """Algorithmic bytes per node and step of a D3Q15 box whose runs take
+    `calls` calls per pass over memory (Lattice.pass_info): pairs of passes,
+    and the rest one call per launch."""
     once = 2 * 15 * slot_bytes
-    cached = slot_bytes == 8 and 128e6 < 15 * 8 * L ** 3 <= 256e6
-    if slot_bytes == 2 or L < 84 or cached or os.environ.get("LBMC_PASS") == "0":
-        return once
-    paired = steps // 4 * 4
-    return once * (paired / 2 + steps - paired) / steps
+    passed = steps // (2 * calls) * (2 * calls)
+    return once * (passed / calls + steps - passed) / steps
 
 
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "step_d3q15_f32_256_traffic.json")
@@ -220,12 +216,12 @@ def main():
     lat.step(t_next, True)
     rho, u = lat.get_macros()
     finite = bool(np.all(np.isfinite(rho)) and np.all(np.isfinite(u)))
+    bytes_node = step_bytes(4, args.steps, lat.pass_info()["calls"])  # all-fluid lattice: no mask read
     lat.close()
     twin.close()
 
     ms_step = ms / args.steps
     mlups = N * args.steps / (ms * 1e-3) / 1e6
-    bytes_node = step_bytes(4, args.steps, L)  # all-fluid lattice: no mask read
     achieved = bytes_node * N / (ms_step * 1e-3) / 1e9
     log(f"bench: {ms_step:.4f} ms/step, {mlups:.0f} MLUPS, {achieved:.0f} GB/s algorithmic, "
         f"wall {wall:.3f} s, finite={finite}")
@@ -248,7 +244,7 @@ def main():
             v.time_steps(0, args.warmup, 0)
             vms = v.time_steps(args.warmup, vsteps, 0)
             vtwin.close()
-            vb = step_bytes(8 if st == lbmc.FP64 else 2, vsteps, L)
+            vb = step_bytes(8 if st == lbmc.FP64 else 2, vsteps, v.pass_info()["calls"])
             variants[lbmc.STORAGE_NAMES[st]] = {
                 "MLUPS": round(N * vsteps / (vms * 1e-3) / 1e6, 1),
                 "ms_per_step": round(vms / vsteps, 5),
