@@ -133,11 +133,16 @@ lbmc_status lbmc_step(lbmc_ctx *ctx, long long t, int store_macros);
 
 /* nsteps calls with t = t0 .. t0+nsteps-1; macros are stored on the calls
  * where (t+1) % store_every == 0 (store_every <= 0: never).  Lattices whose
- * calls the library runs several at a time (D2Q9 without sf boundaries; D3Q15
- * BGK lattices of fluid and solid nodes with FP64 or FP32 storage) hold
- * a second population array from lbmc_set_fields on, taken only while half
- * of the device's memory stays free and given back when a later allocation
- * of the library does not fit; the results do not depend on it. */
+ * calls the library runs several at a time (D2Q9 without sf boundaries, in 16
+ * bits up to 2^20 nodes; D3Q15 lattices of fluid and solid nodes from about
+ * 6e5 on with FP64 or FP32 storage, but FP32 MRT with LBMC_FIX_D3Q15_MINV and
+ * forcing and FP64 ones whose populations take 128 to 256 MB; lbmc_pass_info)
+ * hold a second population array from lbmc_set_fields on, taken only while
+ * half of the device's memory stays free and given back when a later
+ * allocation of the library does not fit (not of other code in the process, and not while
+ * launches of that lattice are being issued); the results do not depend on
+ * it.  Runs of fewer than 4 calls, or of fewer between those that store the
+ * macros of a lattice with prescribed values, take one call per launch. */
 lbmc_status lbmc_run(lbmc_ctx *ctx, long long t0, int nsteps, int store_every);
 
 /* How lbmc_run takes a lattice's calls: *calls per pass over memory, in tiles
@@ -165,12 +170,12 @@ lbmc_status lbmc_set_f(lbmc_ctx *ctx, const double *const *f);
  * reference: it is for callers that cannot allocate device memory (code
  * between graph captures, tight serving or checkpoint loops, harnesses that
  * forbid hipMalloc).  lbmc_get_f allocates an N-double conversion buffer on
- * every call unless the storage is FP64; this variant converts through a fixed 8 MiB device array
- * (1,048,576 doubles, one per GPU for the life of the process), one chunk of
- * at most that many slots of one direction at a time, so lattices of any
- * size are read with the same results, bit for bit.  Calls that overlap on
- * one GPU (other threads, other contexts on the same device) share the array
- * and race: serialise them. */
+ * every call unless the storage is FP64; this variant converts through a
+ * fixed 8 MiB device array (1,048,576 doubles, one per GPU for the life of the
+ * process), one chunk of at most that many slots of one direction at a time,
+ * so lattices of any size are read with the same results, bit for bit.  Calls
+ * that overlap on one GPU (other threads, other contexts on the same device)
+ * share the array and race: serialise them. */
 lbmc_status lbmc_get_f_noalloc(lbmc_ctx *ctx, double *const *f);
 
 /* E = sum_n 1/2 rho |u|^2 over the stored macro arrays (the energy functor
@@ -273,18 +278,19 @@ lbmc_status lbmc_set_closure_shift(lbmc_ctx *ctx, double dtau);
 /* ---- Batches of lattices ---------------------------------------------------
  *
  * Steps an ensemble of independent lattices of different sizes together:
- * D2Q9 members in 32 or 64 bits take several calls per launch (as lbmc_run
- * does); otherwise one persistent launch per time step covers every member's
- * nodes, and runs are replayed from a captured HIP graph.  The reference steps one lattice
- * per process (LBM-C/index.cu:102-108 calling iterate, :284-313); a batch is
- * an addition.  Members are contexts made by lbmc_create and set up as usual
+ * D2Q9 members in 32 or 64 bits take several calls per launch where that
+ * pays, as lbmc_run does; otherwise one persistent launch per time step covers
+ * every member's nodes, and runs are replayed from a captured HIP graph.  The
+ * reference steps one lattice per process (LBM-C/index.cu:102-108 calling
+ * iterate, :284-313); a batch is an addition.  Members are contexts made by lbmc_create and set up as usual
  * (fields and initial state); they share lattice type, storage and device,
  * may differ in size, collision type, forcing, tau and boundary codes, and
  * may not use sf boundaries or direction arrays of 4 GiB or more
  * (LBMC_ERR_UNSUPPORTED).  Members with the learned closure share one
  * model and band; each keeps its own evaluation interval, on the schedule
- * of lbmc_run.  Members must outlive the batch; their state is read at every
- * lbmc_batch_run, and lbmc_get_* on a member reads what the batch computed.
+ * of lbmc_run.  Members must outlive the batch; their state, a closure
+ * switched on or off included, is read at every lbmc_batch_run, and
+ * lbmc_get_* on a member reads what the batch computed.
  */
 typedef struct lbmc_batch lbmc_batch;
 

@@ -6,9 +6,9 @@
 // with the recorded tau up to the next evaluation.
 //
 // Bound by vector-instruction issue, like the single-lattice passes.  64
-// uneven channels (11.2 M nodes, FP32, MRT and BGK with forcing): 172 -> 108
+// uneven channels (11.2 M nodes, FP32, MRT and BGK with forcing): 172 -> 102-108
 // us per call (five calls a pass, 1.29 nodes computed per node owned);
-// with the BGK members' closure evaluated every 8th call 194 -> 142 us.
+// with the BGK members' closure evaluated every 8th call 194 -> 134-140 us.
 // Tiles are listed by collision variant, so that blocks that run together
 // share the instruction cache.
 #pragma once

@@ -33,7 +33,7 @@ hipError_t launch_tile_fp16s(const KernelKey &k, int size, const StepArgs<float>
 hipError_t launch_tile_bf16s(const KernelKey &k, int size, const StepArgs<float> &a, const TilePass &p, int tiles,
                              hipStream_t s);
 
-// two calls of a D3Q15 lattice (BGK family) in one pass, march_<storage>.hip
+// two calls of a D3Q15 lattice in one pass (march_takes), march_<storage>.hip
 hipError_t launch_march_fp64(const KernelKey &k, const StepArgs<double> &a, const MarchPass &p, hipStream_t s);
 hipError_t launch_march_fp32(const KernelKey &k, const StepArgs<float> &a, const MarchPass &p, hipStream_t s);
 

@@ -4,10 +4,10 @@
 // take pieces in turn: an asynchronous copy into the thread's own pinned slot,
 // then the (widening) copy out of it, so the link, the page faults and the
 // conversion overlap.  Reading rho and u of a 256^3 FP32 lattice (268 MB over
-// the link, 537 MB of doubles) took 127 ms by hipMemcpy and a loop, and takes
-// 12 ms; the 15 populations of a 131x97x75 FP64 lattice (114 MB) in and out,
-// with rho and u, 28 and 4.5 ms; 12 bytes of one node 33 and 17 us, by one wait
-// instead of three.
+// the link, 537 MB of doubles) took 80-127 ms by hipMemcpy and a loop, and takes
+// 9-12 ms; of a 131x97x75 FP64 lattice the 15 populations (114 MB) in took 4.8
+// ms, out 15.1 ms, rho and u 2.5 ms, and take 3.1, 3.4 and 1.0 ms; 12 bytes of
+// one node 33 and 17 us, by one wait instead of three.
 #include "host_copy.hpp"
 
 #include <algorithm>

@@ -27,10 +27,10 @@
 // bytes per FP32 node and call; five calls per pass move (36 x 1.7 + 36) / 5
 // = 20, and recompute 1.2-1.35 times the nodes, which the arithmetic units
 // had to spare.  Measured (MI355X, us per call, one call per launch ->
-// passes): FP32 BGK 4096 x 4096 221 -> 94 (tiles of 64 x 32, M = 4: 180 k
-// MLUPS), FP32 MRT 2048 x 1024 22.2 -> 15.0, FP64 MRT 46.2 -> 29.4 (32 x
-// 32, M = 2); small lattices also save the launches, FP64 256 x 64 4.1 ->
-// 1.7.  Two blocks of 72 KB LDS per CU hide one block's loads and stores
+// passes): FP32 BGK box 4096 x 4096 224 -> 90 (tiles of 64 x 32, M = 4: 187 k
+// MLUPS), forced channel 224 -> 105; MRT between pressure faces 2048 x 1024
+// FP32 25.1 -> 19.3, FP64 46.9 -> 31.3 (32 x 32, M = 3); small lattices also
+// save the launches, FP64 256 x 64 3.8 -> 1.9.  Two blocks of 72 KB LDS per CU hide one block's loads and stores
 // under the other's arithmetic: one block of 144 KB (64 x 64 tiles, less
 // recomputation) is 2-20 % slower.
 #pragma once

@@ -148,20 +148,20 @@ inline double tile_estimate(const TilePlan &q, int slot_bytes, int ncu, int call
 
 // The plan with the smallest estimate (within 10 % of the best of all
 // shapes on ten lattices from 64 x 48 to 3392 x 3392, three formats).  In 32
-// and 64 bits it beats one call per launch at every size (us per call, one
-// call per launch -> passes: 256 x 64 FP64 4.1 -> 1.7, 600 x 300 FP32 6.4 ->
-// 3.2, 2048 x 1024 FP32 25.3 -> 15.7, FP64 46.8 -> 39.6, 3392 x 3392 FP32
-// 161 -> 78).  The 16-bit one-call kernels move half of FP32's bytes and are
+// and 64 bits it beats one call per launch at every size (us per call of a
+// forced BGK channel, one call per launch -> passes: 256 x 64 FP64 3.8 -> 1.9,
+// 600 x 300 FP32 6.2 -> 3.2, 2048 x 1024 FP32 25.2 -> 15.1, FP64 46.4 -> 34.0,
+// 3392 x 3392 FP32 160 -> 68).  The 16-bit one-call kernels move half of FP32's bytes and are
 // bound by the same arithmetic plus the conversions, so passes win only
-// where launches count: 64 x 48 3.4 -> 1.2, 1500 x 400 11.6 -> 8.0, 2786 x
+// where launches count: 64 x 48 3.3 -> 1.2, 1500 x 400 11.3 -> 7.9, 2786 x
 // 681 equal, 3392 x 3392 80 -> 92; hence the line at 2^20 nodes.
 // Lattices with nodes of other classes than fluid and solid (boundary,
 // prescribed or porous: plain false) take tiles of up to 512 nodes below 1.5e6
 // nodes in 16 and 32 bits: a tile that holds such nodes takes longer, and of a
 // few rounds of large tiles the last waits for it (MRT between pressure faces,
-// tiles of 2048 -> 512 nodes: FP32 512 x 512 7.4 -> 5.4, 1148 x 450 9.3 -> 7.5,
-// 1222 x 1000 15.4 -> 13.4, 1400 x 1400 19.6 against 19.0-19.9; FP16S 800 x 640
-// 14.6 -> 8.4, one call per launch 11.9; 64 bits hold 1024 and gain 0-5 %).
+// tiles of 2048 -> 512 nodes: FP32 512 x 512 7.4 -> 5.4, 1148 x 450 9.3 -> 7.4,
+// 1222 x 1000 15.4 -> 13.0, 1400 x 1400 19.6 against 19.0-19.9; FP16S 800 x 640
+// 14.6 -> 8.1, one call per launch 11.7; 64 bits hold 1024 and gain 0-5 %).
 // M up to 7: deeper passes of the small tiles recompute more than they save.
 // calls: the plan for passes of that many (0: the best of all).
 inline TilePlan plan_tiles(int Lx, int Ly, int slot_bytes, int ncu, bool plain, int calls = 0)
