@@ -101,7 +101,7 @@ inline bool tile_shape(int Lx, int Ly, int size, int W, int H, int M, TilePlan &
 // Runs of fewer calls go one call per launch (us for 3 calls, one by one and in
 // passes of one and two: 2048 x 1024 FP64 143, 185, FP32 76, 86; 1148 x 450
 // FP16S 29, 40); with 4 passes are ahead in every format and size that has them
-// (1.04 to 1.8 times).
+// (1.01 to 1.7 times).
 constexpr int kMinPassRun = 4;
 
 // Passes of a run of len calls, K at most in each: an even number, so that the
